@@ -1,6 +1,11 @@
-// mhc_pre_clamp_sinkhorn forward, one kernel per call.
+// mhc_pre_clamp_sinkhorn forward.
 //
 // Semantics: mhc_pre_clamp_sinkhorn_ref, src/mhc_pre_clamp_sinkhorn.py:974-1022.
+//
+// bf16 x and phi with 16-byte aligned rows run the LDS-pipelined kernels below
+// (or the single pass, pre_fwd_coop.hpp); every other type and alignment the
+// general contraction (pre_fwd_gen.hpp).  pre_fwd_kernel, one kernel per call,
+// runs where the caller's workspace holds neither's sums.
 //
 // A block (4 waves) owns a tile of 64 tokens (4 row blocks of 16):
 //   1. contraction  acc[t,m] = sum_k x[t,k] * phi[m,k]  (k = n*D + d) on bf16
@@ -60,6 +65,11 @@ struct PreFwdArgs {
   float* part_ssq;
   float* pre_ws;
   float* inv_ws;
+  // general contraction (pre_fwd_gen.hpp): phi in its own dtype, stages per
+  // tile, stages per block and tokens per tile (gen_w == 0: not that form)
+  const void* phi_raw;
+  int gen_nst, gen_tt;
+  int64_t gen_w;
   // single-pass form: its status word (nonzero when a bounded wait timed
   // out); the finalize kernel then writes NaN to every output of the call
   // and copies the word to status_out (the caller's, may be null)
@@ -854,6 +864,14 @@ __global__ __launch_bounds__(kKsThreads) void pre_fwd_ks8_kernel(PreFwdArgs a) {
   }
 }
 
+// The slots of a token's sums: `nsplit` of them, or, after the general
+// contraction, the blocks whose runs touch the token's tile.
+__device__ __forceinline__ int fwd_slots(const PreFwdArgs& a, int64_t tok, int nsplit) {
+  if (!a.gen_w) return nsplit;
+  const int64_t tile = tok / a.gen_tt;
+  return (int)(((tile + 1) * a.gen_nst - 1) / a.gen_w - tile * a.gen_nst / a.gen_w) + 1;
+}
+
 // ---- split-K form, kernels 2 and 3 -----------------------------------------
 // Kernel 2: one N x N lane group per token sums the splits' partials in split
 // order, then computes inv_rms, mixes, heads, clamp and Sinkhorn exactly as
@@ -871,8 +889,9 @@ __global__ __launch_bounds__(kFwdThreads) void pre_fwd_finalize_kernel(PreFwdArg
   // unconditional loads (lanes e >= 2N sum a column they never use), so the
   // unrolled iterations issue together instead of waiting one by one
   const int eh = e < 2 * N ? e : 0;
+  const int ns = fwd_slots(a, tk, nsplit);
 #pragma unroll 8
-  for (int s = 0; s < nsplit; ++s) {
+  for (int s = 0; s < ns; ++s) {
     const int64_t row = (int64_t)s * T + tk;
     ssq += a.part_ssq[row];
     acc_l += a.part[row * M + 2 * N + e];
@@ -1081,6 +1100,7 @@ static FwdSplitPlan fwd_split_plan(int64_t T, int N, int D) {
 }  // namespace mhc
 
 #include "pre_fwd_coop.hpp"
+#include "pre_fwd_gen.hpp"
 
 namespace mhc {
 
@@ -1186,6 +1206,21 @@ static int dispatch_pre_fwd(int N, const PreFwdArgs& a, bool vec, hipStream_t st
   return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_fwd: N=%d not supported (4, 8)", N);
 }
 
+template <int N>
+static int dispatch_pre_fwd_gen_x(int32_t x_dtype, const PreFwdArgs& a, int32_t phi_dtype, int64_t chunk,
+                                  void* workspace, hipStream_t st) {
+  switch (x_dtype) {
+    case MHC_DTYPE_BF16: return launch_pre_fwd_gen<N, bf16_t>(a, phi_dtype, chunk, workspace, st);
+    case MHC_DTYPE_F16: return launch_pre_fwd_gen<N, f16_t>(a, phi_dtype, chunk, workspace, st);
+    default: return launch_pre_fwd_gen<N, float>(a, phi_dtype, chunk, workspace, st);
+  }
+}
+static int dispatch_pre_fwd_gen(int N, int32_t x_dtype, const PreFwdArgs& a, int32_t phi_dtype, int64_t chunk,
+                                void* workspace, hipStream_t st) {
+  return N == 4 ? dispatch_pre_fwd_gen_x<4>(x_dtype, a, phi_dtype, chunk, workspace, st)
+                : dispatch_pre_fwd_gen_x<8>(x_dtype, a, phi_dtype, chunk, workspace, st);
+}
+
 }  // namespace mhc
 
 using namespace mhc;
@@ -1207,8 +1242,12 @@ static size_t pre_fwd_ws_min(int64_t T, int32_t N, int32_t D, int32_t phi_dtype)
 
 // With room for the single-pass form where it applies (N = 4, bf16 phi).
 extern "C" size_t mhc_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, int32_t phi_dtype) {
-  const size_t base = pre_fwd_ws_min(T, N, D, phi_dtype);
-  if (phi_dtype != MHC_DTYPE_BF16) return base;
+  size_t base = pre_fwd_ws_min(T, N, D, phi_dtype);
+  if (N != 4 && N != 8) return base;
+  if (phi_dtype != MHC_DTYPE_BF16 || (int64_t)N * D % 8) {  // the general form's sums
+    const size_t gen = D > 0 && T > 0 ? gen_ws_bytes(T, N, D) : 0;
+    return gen > base ? gen : base;
+  }
   const size_t coop = coop_ws_bytes(T, N, D);
   return coop && kPreFwdWsBase + coop > base ? kPreFwdWsBase + coop : base;
 }
@@ -1303,9 +1342,6 @@ extern "C" int mhc_pre_fwd_ex(const void* x, int32_t x_dtype, const void* phi, i
 
   PreFwdArgs a{};
   a.x = x;
-  int rc = prepare_phi_planes(phi, phi_dtype, M, K, workspace, workspace_bytes, &a.phi, &a.phi_ld,
-                              &a.phi_plane_stride, &a.phi_planes, st);
-  if (rc) return rc;
   a.alpha = alpha;
   a.base = base;
   a.norm_eps = norm_eps;
@@ -1326,6 +1362,17 @@ extern "C" int mhc_pre_fwd_ex(const void* x, int32_t x_dtype, const void* phi, i
   a.D = D;
   a.status_out = status;
   const bool vec = (D % 8 == 0) && aligned16(x) && aligned16(y) && (!x_scaled || aligned16(x_scaled));
+  if (x_dtype < 0 || x_dtype > 2) return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_fwd: x dtype %d not supported", x_dtype);
+  if (phi_dtype < 0 || phi_dtype > 2) return set_error(MHC_ERR_UNSUPPORTED, "phi dtype %d not supported", phi_dtype);
+  const bool streaming = x_dtype == MHC_DTYPE_BF16 && phi_dtype == MHC_DTYPE_BF16 && vec && K % 8 == 0 && aligned16(phi);
+  const int64_t chunk = streaming || !workspace ? 0 : gen_chunk(T, N, D, workspace_bytes);
+  if (chunk > 0) {
+    a.phi_raw = phi;
+    return dispatch_pre_fwd_gen(N, x_dtype, a, phi_dtype, chunk, workspace, st);
+  }
+  int rc = prepare_phi_planes(phi, phi_dtype, M, K, workspace, workspace_bytes, &a.phi, &a.phi_ld,
+                              &a.phi_plane_stride, &a.phi_planes, st);
+  if (rc) return rc;
   const size_t y_ws = fwd_y_ws_bytes(T, N), ha_ws = heads_apart_bytes(T, N);
   const size_t dma_ws = kPreFwdWsBase + (ha_ws > y_ws ? ha_ws : y_ws);
   if (fwd_dma_usable(a, N, x_dtype == MHC_DTYPE_BF16, vec) && workspace && workspace_bytes >= dma_ws)

@@ -1,0 +1,125 @@
+"""The pre forward's general contraction and finish kernels (csrc/pre_fwd_gen.hpp)
+at the edges of their tiles, runs and pieces, against the float64 oracle.
+
+Tolerances as in test_gpu_pre.py; with fp32 x and phi the three-plane products
+keep the mixes within 1e-4 and y is fp32, rtol / atol 1e-5."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import FlagOS_mhc as m
+from FlagOS_mhc import _lib
+from test_gpu_post import DEV, _subset, assert_close
+from test_gpu_pre import FWD_KEYS, _oracle_fwd, check_fwd, pre_inputs
+
+pytestmark = pytest.mark.gpu
+
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+CASES = [
+    # T, N, D, x, phi: 16-token tiles (T <= 64), one stage a tile or several
+    # tiles a block; K and D that end inside a stage, a 32-column step, an
+    # 8-element group and a 4-element piece
+    (1, 4, 7168, BF, F32), (1, 4, 64, F32, F32), (2, 8, 9, HF, F32), (16, 4, 1003, HF, HF), (17, 8, 200, BF, F32),
+    (64, 4, 4096, BF, F32), (64, 8, 1031, F32, F32), (33, 4, 3, BF, BF), (5, 8, 2048, BF, F32),
+    # 128-token tiles: one token past a tile, runs that end inside a tile
+    # (65 tiles), the finish kernel's largest T and one more
+    (65, 4, 256, F32, F32), (128, 4, 1003, HF, HF), (129, 4, 515, BF, F32), (777, 4, 4096, BF, F32),
+    (2048, 4, 130, HF, F32), (2049, 4, 1003, HF, HF), (8193, 4, 3584, BF, F32), (2049, 8, 517, BF, F32),
+    (3000, 8, 1024, F32, F32), (1025, 8, 640, HF, HF), (1030, 8, 333, HF, BF), (1030, 4, 1030, F32, BF),
+    (2500, 4, 6001, F32, F32), (66000, 4, 24, BF, F32),
+]
+
+
+def _kw(clamp=10.0, iters=20):
+    return dict(norm_eps=1e-6, hc_eps=1e-6, clamp_min=-clamp, clamp_max=clamp, iter_times=iters)
+
+
+def _check(x, phi, alpha, base, kw, what):
+    T, dtype = x.shape[0], x.dtype
+    out = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, need_backward=True, **kw)
+    torch.cuda.synchronize()
+    idx = _subset(T, k=48, seed=T)
+    want = _oracle_fwd(idx, x, phi, alpha, base, kw)
+    check_fwd(out, want, dtype, idx, what)
+    if dtype == F32:
+        assert_close(out["y"][idx], want["y"], 1e-5, 1e-5, what + " y")
+    assert_close(out["x_scaled"][idx], want["x_scaled"], 1e-5, 1e-6, what + " x_scaled")
+    small = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, **kw)
+    for k in small:
+        assert torch.equal(small[k], out[k]), what + " " + k
+    return out
+
+
+@pytest.mark.parametrize("T,N,D,dtype,phi_dtype", CASES)
+def test_general_contraction(T, N, D, dtype, phi_dtype):
+    print(f"[pre_fwd general] T={T} N={N} D={D} {dtype} phi={phi_dtype}", flush=True)
+    x, phi, alpha, base, *_ = pre_inputs(T, N, D, dtype, phi_dtype, seed=T + D)
+    _check(x, phi, alpha, base, _kw(iters=7 if D % 2 else 20), f"T={T} N={N} D={D}")
+
+
+@pytest.mark.parametrize("dtype,phi_dtype,T", [(BF, F32, 70), (HF, HF, 3), (F32, F32, 200), (BF, BF, 300)])
+def test_unaligned_bases(dtype, phi_dtype, T):
+    """x, phi and the gates as views one element into their storage."""
+    N, D = 4, 520
+    x, phi, alpha, base, *_ = pre_inputs(T, N, D, dtype, phi_dtype, seed=5)
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, device=DEV, dtype=t.dtype)
+        buf[1:] = t.reshape(-1)
+        return buf[1:].view(t.shape)
+
+    print(f"[pre_fwd general] unaligned {dtype} {phi_dtype} T={T}", flush=True)
+    got = _check(shifted(x), shifted(phi), alpha, base, _kw(), "unaligned")
+    if (dtype, phi_dtype) != (BF, BF):  # the aligned bf16 pair has a kernel of its own
+        want = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, need_backward=True, **_kw())
+        for k in want:
+            assert torch.equal(got[k], want[k]), k
+
+
+def test_inf_and_nan_rows_stay_in_their_rows():
+    """An infinite or NaN activation spoils its own token only (D ends inside
+    a stage: the columns past it must not meet the value)."""
+    x, phi, alpha, base, *_ = pre_inputs(140, 4, 133, BF, F32, seed=3)
+    clean = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, **_kw())
+    x = x.clone()
+    x[3, 3, 132], x[137, 0, 0] = float("inf"), float("nan")
+    out = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, **_kw())
+    torch.cuda.synchronize()
+    keep = torch.ones(140, dtype=torch.bool, device=DEV)
+    keep[[3, 137]] = False
+    for k in clean:
+        assert torch.equal(out[k][keep], clean[k][keep]), k
+    assert not torch.isfinite(out["y"][137].float()).any()
+
+
+@pytest.mark.parametrize("share,T", [(1.0, 9000), (0.6, 9000), (0.0, 300)])
+def test_workspace_smaller_than_asked(share, T):
+    """mhc_pre_fwd with less workspace than mhc_pre_fwd_workspace_size: the
+    tokens in chunks that fit, or the form that keeps no sums in memory; the
+    same results to rounding."""
+    N, D = 4, 260
+    x, phi, alpha, base, *_ = pre_inputs(T, N, D, BF, F32, seed=9)
+    lib, M = _lib.load(), 24
+    full = lib.mhc_pre_fwd_workspace_size(T, N, D, 0)
+    planes = 3 * M * N * D * 2
+    want = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, need_backward=True, **_kw())
+    f32 = dict(device=DEV, dtype=F32)
+    o = {"y": torch.empty(T, D, device=DEV, dtype=BF), "post_out": torch.empty(T, N, **f32),
+         "comb_frag": torch.empty(T, N, N, **f32), "inv_rms": torch.empty(T, **f32),
+         "mixes": torch.empty(T, M, **f32), "h_res_logits": torch.empty(T, N, N, **f32),
+         "pre": torch.empty(T, N, **f32), "x_scaled": torch.empty(T, N * D, **f32)}
+    size = max(int(full * share), planes)
+    ws = torch.empty(size, dtype=torch.uint8, device=DEV)
+    print(f"[pre_fwd general] workspace {size} of {full}", flush=True)
+    rc = lib.mhc_pre_fwd(x.data_ptr(), 1, phi.data_ptr(), 0, alpha.data_ptr(), base.data_ptr(), 1e-6, 1e-6, -10.0,
+                         10.0, 20, *(t.data_ptr() for t in o.values()), ws.data_ptr(), size, T, N, D,
+                         torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "mhc_pre_fwd")
+    torch.cuda.synchronize()
+    assert_close(o["y"], want["y"].double().cpu().numpy(), 2e-2, 2e-2, "y")
+    for k in FWD_KEYS:
+        assert_close(o[k], want[k].double().cpu().numpy(), 1e-4, 1e-5, k)
+    assert_close(o["x_scaled"], want["x_scaled"].double().cpu().numpy().reshape(T, N * D), 1e-5, 1e-6, "x_scaled")
