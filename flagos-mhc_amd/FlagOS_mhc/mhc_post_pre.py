@@ -76,7 +76,8 @@ def mhc_post_pre_clamp_sinkhorn(
         pre = torch.empty((T, N), **f32)
     if T > 0:
         lib = _lib.load()
-        ws_bytes = int(lib.mhc_post_pre_fwd_workspace_size(T, N, D, pcode))
+        # x that is not bf16 runs the general form, whose workspace is that of an fp32 phi
+        ws_bytes = int(lib.mhc_post_pre_fwd_workspace_size(T, N, D, pcode if xf.dtype == torch.bfloat16 else 0))
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
         # the shapes a single pass can take report its bounded waits into a
         # status word, as the pre forward's

@@ -15,12 +15,11 @@
 //   -> grad_mixes (T,M) and scale[t] = -inv^2 * <grad_mixes, mixes> / (N*D)
 //   (because <x, grad_mixes @ phi> = <grad_mixes, mixes> / inv), plus a
 //   per-block partial of grad_alpha / grad_base (fixed summation order).
-// Kernel B (pre_bwd_main_kernel), a block per (256 k-columns, token split):
-//   gs = grad_mixes @ phi on MFMA (A = phi^T rows kept in registers,
-//   B = grad_mixes rows from LDS), then
-//   grad_x = grad_y * pre[n] + inv * gs + scale * x, written once;
-//   grad_phi partial += (grad_mixes * inv)^T @ x on MFMA over 32-token
-//   sub-tiles staged in LDS.
+// Kernel B, a block per (columns, token split): gs = grad_mixes @ phi on MFMA,
+//   grad_x = grad_y * pre[n] + inv * gs + scale * x, written once, and
+//   grad_phi partial += (grad_mixes * inv)^T @ x on MFMA over 16-token tiles:
+//   pre_bwd_dma_kernel for bf16 rows of 16-byte pieces, pre_bwd_gen_kernel
+//   (pre_bwd_gen.hpp) for every other type, width and alignment.
 // Kernels C: deterministic reductions of the grad_phi split partials and of
 // the grad_alpha / grad_base block partials (no atomics anywhere).
 #include <type_traits>
@@ -34,8 +33,6 @@ namespace mhc {
 
 constexpr int kBwdTile = 16;
 constexpr int kBwdThreads = 256;
-constexpr int kMainKC = 256;  // k columns per main-kernel block (all N streams x KC/N widths)
-constexpr int kMainTS = 32;   // tokens per main-kernel sub-tile
 constexpr int kMaxSplits = 16;
 
 // ---------------------------------------------------------------------------
@@ -102,7 +99,7 @@ constexpr int kGpreCols = kBwdThreads * 8;
 // 2^32 work-items of a dispatch at any T.
 constexpr int64_t kGpreGridT = 65536;
 
-template <int N, typename S, bool VEC>
+template <int N, typename S>
 __global__ __launch_bounds__(kBwdThreads) void pre_bwd_gpre_kernel(const void* xv, const void* gyv, float* part,
                                                                    int64_t T, int D) {
   __shared__ float red[kBwdThreads / kWave][N];
@@ -110,15 +107,14 @@ __global__ __launch_bounds__(kBwdThreads) void pre_bwd_gpre_kernel(const void* x
   const S* __restrict__ gy = static_cast<const S*>(gyv);
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
   const int64_t d = (int64_t)blockIdx.y * kGpreCols + tid * 8;
-  const bool ok = d < D;
   for (int64_t tok = blockIdx.x; tok < T; tok += gridDim.x) {  // uniform over the block
     float acc[N];
     float g8[8];
-    load8f<S, VEC>(gy + tok * D, d, D, ok, g8);
+    load8u(gy + tok * D, d, D, g8);
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       float x8[8];
-      load8f<S, VEC>(x + (tok * N + n) * D, d, D, ok, x8);
+      load8u(x + (tok * N + n) * D, d, D, x8);
       acc[n] = 0.f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[n] = fmaf(g8[i], x8[i], acc[n]);
@@ -246,7 +242,7 @@ __global__ __launch_bounds__(kWave * kGpreDmaWaves) void pre_bwd_gpre_dma_kernel
 // mixes[0..3], inv_rms, scale without the pre head, 0, 0} carries what the
 // single-pass kernel needs to add them (grad_mixes[t, n] = grad_pre[t, n] *
 // alpha[0] * sp(1 - sp)).
-template <int N, typename S, bool VEC, bool SP = false>
+template <int N, typename S, bool SP = false>
 __global__ __launch_bounds__(kBwdThreads) void pre_bwd_small_kernel(PreBwdSmallArgs a) {
   static_assert(!SP || N == 4, "single-pass records hold four streams");
   using PD = PreDims<N>;
@@ -287,11 +283,11 @@ __global__ __launch_bounds__(kBwdThreads) void pre_bwd_small_kernel(PreBwdSmallA
       if (tok < a.T) {
         for (int64_t d = (int64_t)lane * 8; d < D; d += kWave * 8) {
           float g8[8];
-          load8f<S, VEC>(gy + tok * D, d, D, true, g8);
+          load8u(gy + tok * D, d, D, g8);
 #pragma unroll
           for (int n = 0; n < N; ++n) {
             float x8[8];
-            load8f<S, VEC>(x + (tok * N + n) * D, d, D, true, x8);
+            load8u(x + (tok * N + n) * D, d, D, x8);
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[n] = fmaf(g8[i], x8[i], acc[n]);
           }
@@ -437,289 +433,24 @@ __global__ __launch_bounds__(kBwdThreads) void pre_bwd_small_kernel(PreBwdSmallA
 // ---------------------------------------------------------------------------
 // Kernel B
 // ---------------------------------------------------------------------------
-struct PreBwdMainArgs {
-  const void* x;
-  const void* gy;
-  const uint16_t* phiT;  // [P][K][MP32]
-  int64_t phiT_plane_stride;
-  int phi_planes;
-  const float* gm;
-  const float* inv_rms;
-  const float* pre;
-  const float* scale;
-  void* gx;
-  float* gphi_part;  // [nsplit][M][K]
-  int64_t T;
-  int D;
-  int64_t tok_per_split;
-};
-
-template <typename S> struct Raw { typedef uint16_t type; };
-template <> struct Raw<float> { typedef float type; };
-
-template <typename S> __device__ __forceinline__ float raw_to_f32(typename Raw<S>::type v) {
-  return Store<S>::to_f32(v);
-}
-template <> __device__ __forceinline__ float raw_to_f32<float>(float v) { return v; }
-
-// 8 raw elements of a row (element-wise with bound `lim` unless VEC)
-template <typename S, bool VEC>
-__device__ __forceinline__ void copy8_to_lds(const S* src, int64_t lim, bool ok,
-                                             typename Raw<S>::type* dst) {
-  typedef typename Raw<S>::type R;
-  if constexpr (VEC) {
-    if constexpr (sizeof(S) == 2) {
-      const u32x4 v = (ok && lim >= 8) ? ld16nt(src) : zero4();
-      st16(dst, v);
-    } else {
-      u32x4 v0 = zero4(), v1 = zero4();
-      if (ok && lim >= 8) {
-        v0 = ld16nt(src);
-        v1 = ld16nt(src + 4);
-      }
-      st16(dst, v0);
-      st16(dst + 4, v1);
-    }
-  } else {
-    const R* s = reinterpret_cast<const R*>(src);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) dst[i] = (ok && i < lim) ? s[i] : (R)0;
-  }
-}
-
-template <int N, typename S, bool VEC>
-__global__ __launch_bounds__(256) void pre_bwd_main_kernel(PreBwdMainArgs a) {
-  using PD = PreDims<N>;
-  typedef typename Raw<S>::type R;
-  constexpr int M = PD::M, MT = PD::MT, MP = PD::MP, MK = PD::MK, MP32 = PD::MP32;
-  constexpr int KC = kMainKC, DC = KC / N, TS = kMainTS;
-  constexpr int XP = XGroup<S>::PLANES;
-  constexpr int XPITCH = KC + 8, GPITCH = DC + 8, MPITCH = MP32 + 8, TPITCH = TS + 8;
-
-  __shared__ __attribute__((aligned(16))) R xs[TS][XPITCH];
-  __shared__ __attribute__((aligned(16))) R gys[TS][GPITCH];
-  __shared__ __attribute__((aligned(16))) uint16_t gmS[2][TS][MPITCH];
-  __shared__ __attribute__((aligned(16))) uint16_t gT[2][MP][TPITCH];
-  __shared__ float pre_sh[TS][N];
-  __shared__ float inv_sh[TS], scale_sh[TS];
-
-  const S* __restrict__ x = static_cast<const S*>(a.x);
-  const S* __restrict__ gy = static_cast<const S*>(a.gy);
-  S* __restrict__ gx = static_cast<S*>(a.gx);
-  const int D = a.D;
-  const int64_t K = (int64_t)N * D;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15, kq = lane >> 4;
-  const int d0 = blockIdx.x * DC;
-  const int64_t tbeg = (int64_t)blockIdx.y * a.tok_per_split;
-  const int64_t tend = (tbeg + a.tok_per_split < a.T) ? tbeg + a.tok_per_split : a.T;
-  const int P = a.phi_planes;
-
-  // padding rows/columns of the operand tiles stay zero
-  for (int i = tid; i < 2 * TS * MPITCH; i += 256) (&gmS[0][0][0])[i] = 0;
-  for (int i = tid; i < 2 * MP * TPITCH; i += 256) (&gT[0][0][0])[i] = 0;
-
-  // A operands of gs^T = phi^T-rows x grad_mixes^T: MFMA row rr of k-tile q maps to
-  // wave column 16*(rr/4) + 4*q + rr%4, so each lane's outputs cover 16
-  // consecutive columns.
-  u32x4 aphi[4][MK][2];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int col = wave * 64 + 16 * (r >> 2) + 4 * q + (r & 3);
-    const int n = col / DC, dd = col - (col / DC) * DC;
-    const bool ok = d0 + dd < D;
-    const int64_t kg = (int64_t)n * D + d0 + dd;
-#pragma unroll
-    for (int mk = 0; mk < MK; ++mk)
-#pragma unroll
-      for (int p = 0; p < 2; ++p)
-        aphi[q][mk][p] = (ok && p < P)
-                             ? ld16(a.phiT + p * a.phiT_plane_stride + kg * MP32 + 32 * mk + 8 * kq)
-                             : zero4();
-  }
-
-  floatx4 ph[4][MT];
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) ph[q][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  for (int64_t tb = tbeg; tb < tend; tb += TS) {
-    __syncthreads();  // previous sub-tile fully consumed
-    // ---- stage the sub-tile -------------------------------------------------
-    constexpr int UPT = N * (DC / 8);  // 8-element units per token row chunk
-    for (int u = tid; u < TS * UPT; u += 256) {
-      const int tt = u / UPT, rem = u - (u / UPT) * UPT;
-      const int n = rem / (DC / 8), dd = (rem - (rem / (DC / 8)) * (DC / 8)) * 8;
-      const int64_t tok = tb + tt;
-      copy8_to_lds<S, VEC>(x + (tok * N + n) * D + d0 + dd, (int64_t)D - d0 - dd, tok < tend,
-                           &xs[tt][n * DC + dd]);
-    }
-    for (int u = tid; u < TS * (DC / 8); u += 256) {
-      const int tt = u / (DC / 8), dd = (u - (u / (DC / 8)) * (DC / 8)) * 8;
-      const int64_t tok = tb + tt;
-      copy8_to_lds<S, VEC>(gy + tok * D + d0 + dd, (int64_t)D - d0 - dd, tok < tend, &gys[tt][dd]);
-    }
-    for (int u = tid; u < TS * M; u += 256) {
-      const int tt = u / M, m = u - (u / M) * M;
-      const int64_t tok = tb + tt;
-      const bool ok = tok < tend;
-      const float v = ok ? a.gm[tok * M + m] : 0.f;
-      const float inv = ok ? a.inv_rms[tok] : 0.f;
-      uint32_t hi, lo;
-      split2_bf16(v, hi, lo);
-      gmS[0][tt][m] = (uint16_t)hi;
-      gmS[1][tt][m] = (uint16_t)lo;
-      split2_bf16(v * inv, hi, lo);
-      gT[0][m][tt] = (uint16_t)hi;
-      gT[1][m][tt] = (uint16_t)lo;
-    }
-    for (int u = tid; u < TS * N; u += 256) {
-      const int tt = u / N, n = u - (u / N) * N;
-      const int64_t tok = tb + tt;
-      pre_sh[tt][n] = tok < tend ? a.pre[tok * N + n] : 0.f;
-    }
-    if (tid < TS) {
-      const int64_t tok = tb + tid;
-      inv_sh[tid] = tok < tend ? a.inv_rms[tok] : 0.f;
-      scale_sh[tid] = tok < tend ? a.scale[tok] : 0.f;
-    }
-    __syncthreads();
-
-    // ---- gs and grad_x ---------------------------------------------------------
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int tt = 16 * h + r;
-      floatx4 gs[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) gs[q] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int mk = 0; mk < MK; ++mk) {
-        const u32x4 b0 = *reinterpret_cast<const u32x4*>(&gmS[0][tt][32 * mk + 8 * kq]);
-        const u32x4 b1 = *reinterpret_cast<const u32x4*>(&gmS[1][tt][32 * mk + 8 * kq]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          gs[q] = mfma16x16x32(as_bf16x8(aphi[q][mk][0]), as_bf16x8(b0), gs[q]);
-          gs[q] = mfma16x16x32(as_bf16x8(aphi[q][mk][0]), as_bf16x8(b1), gs[q]);
-          if (P > 1) gs[q] = mfma16x16x32(as_bf16x8(aphi[q][mk][1]), as_bf16x8(b0), gs[q]);
-        }
-      }
-      const int col0 = wave * 64 + 16 * kq;
-      const int n = col0 / DC, dd0 = col0 - (col0 / DC) * DC;
-      const float pn = pre_sh[tt][n], iv = inv_sh[tt], sc = scale_sh[tt];
-      float o[16];
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        const float xv = raw_to_f32<S>(xs[tt][col0 + c]);
-        const float gv = raw_to_f32<S>(gys[tt][dd0 + c]);
-        o[c] = fmaf(sc, xv, fmaf(iv, gs[c >> 2][c & 3], gv * pn));
-      }
-      const int64_t tok = tb + tt;
-      if (tok < tend) {
-        S* dst = gx + (tok * N + n) * D + d0;
-        store8<S, VEC>(dst, dd0, (int64_t)D - d0, o);
-        store8<S, VEC>(dst, dd0 + 8, (int64_t)D - d0, o + 8);
-      }
-    }
-
-    // ---- grad_phi partial += (grad_mixes*inv)^T @ x -------------------------
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int col = wave * 64 + 16 * q + r;
-      float f[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = raw_to_f32<S>(xs[8 * kq + e][col]);
-      u32x4 bx[2];
-      if constexpr (XP == 1) {
-        // bf16: rebuild the operand from raw bits (exact)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          bx[0][i] = (uint32_t)xs[8 * kq + 2 * i][col] | ((uint32_t)xs[8 * kq + 2 * i + 1][col] << 16);
-        bx[1] = zero4();
-      } else {
-        split8(f, bx[0], bx[1]);
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const u32x4 g0 = *reinterpret_cast<const u32x4*>(&gT[0][16 * mt + r][8 * kq]);
-        const u32x4 g1 = *reinterpret_cast<const u32x4*>(&gT[1][16 * mt + r][8 * kq]);
-        ph[q][mt] = mfma16x16x32(as_bf16x8(g0), as_bf16x8(bx[0]), ph[q][mt]);
-        ph[q][mt] = mfma16x16x32(as_bf16x8(g1), as_bf16x8(bx[0]), ph[q][mt]);
-        if constexpr (XP > 1) ph[q][mt] = mfma16x16x32(as_bf16x8(g0), as_bf16x8(bx[1]), ph[q][mt]);
-      }
-    }
-  }
-
-  // ---- write this split's grad_phi partial ---------------------------------
-  float* part = a.gphi_part + (int64_t)blockIdx.y * M * K;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int col = wave * 64 + 16 * q + r;
-    const int n = col / DC, dd = col - (col / DC) * DC;
-    if (d0 + dd >= D) continue;
-    const int64_t kg = (int64_t)n * D + d0 + dd;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int m = 16 * mt + 4 * kq + v;
-        if (m < M) part[(int64_t)m * K + kg] = ph[q][mt][v];
-      }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Kernel B, streaming form (bf16 activations, 16-byte aligned rows)
-//
-// A block has one wave per stream n and owns DW = 16*VC columns d of every
-// stream; it walks 16-token tiles t = split, split + nsplit, ... so every
-// block of the persistent grid gets the same work.  Lane (r = lane%16,
-// q = lane/16) loads, for the 4 tokens 4q..4q+3 of a tile, the VC columns
-// d0 + VC*r.. of x[t, n, :] and grad_y[t, :] (one coalesced load per row),
-// i.e. a 4 x VC bf16 block held in registers:
-//   * grad_phi (MFMA 16x16x16, reduction over the 16 tokens): the block is
-//     transposed in registers (16-bit shuffles inside the lane) so that its
-//     column c is a B operand (4 tokens of one column); A = (grad_mixes*inv)^T
-//     read from token-transposed 16-token tiles.  MFMA instance c covers the
-//     columns VC*r + c, r = 0..15.
-//   * gs = grad_mixes @ phi (MFMA 16x16x32, reduction over m): A = the 16
-//     tokens' grad_mixes rows, B = phi^T rows kept in registers for the whole
-//     kernel.  Output lane (r, q) holds tokens 4q..4q+3 of columns VC*r + c:
-//     exactly the rows of x and grad_y the lane loaded, so
-//     grad_x = grad_y*pre + inv*gs + scale*x is formed and stored in place.
-// No LDS and no barriers: each wave streams independently.  Used for N = 8;
-// N = 4 takes the LDS-pipelined form below.
-// ---------------------------------------------------------------------------
-template <int N> struct StreamCfg {
-  static constexpr int VC = (N == 4) ? 8 : 4;  // columns per lane
-  static constexpr int DW = 16 * VC;           // columns per block and stream
-};
-
 constexpr int kStreamTile = 16;  // tokens per tile (MFMA K of the grad_phi product)
 static_assert(kStreamTile == kBwdTile, "kernel A zero-fills the g tiles of the padding tokens");
 
 struct PreBwdStreamArgs {
-  const bf16_t* x;
-  const bf16_t* gy;
+  const void* x;
+  const void* gy;
   const uint16_t* phiT;  // [P][K][MP32]
   int64_t phiT_plane_stride;
-  int phi_planes;
   const uint16_t* gmP;   // [2][T][MP32]
   int64_t gmP_plane;
   const uint16_t* gTw;   // [ceil(T/16)][MT][64][2][4]
   const float4* coef;    // (T, N) {pre, inv, scale, 0}
-  bf16_t* gx;
-  const bf16_t* gin;     // accumulating form (LDS-pipelined kernel): grad_x = gin + dL/dx
+  void* gx;
+  const void* gin;       // accumulating form: grad_x = gin + dL/dx, or null
   float* gphi_part;      // [nsplit][M][K]
   int64_t T;
   int D;
-  int nsplit;
 };
-
-template <int VD> struct RowVec;
-template <> struct RowVec<4> { typedef u32x4 type; };
-template <> struct RowVec<2> { typedef u32x2 type; };
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
@@ -728,185 +459,16 @@ __device__ __forceinline__ floatx4 mfma16x16x16(const u32x2& a, const u32x2& b, 
                                                   __builtin_bit_cast(short4_t, b), c, 0, 0, 0);
 }
 
-// Operands of one 16-token tile.
-template <int N> struct StreamTile {
-  static constexpr int VC = StreamCfg<N>::VC, VD = VC / 2;
-  typedef typename RowVec<VD>::type Row;
-  Row xr[4], gr[4];                   // x[t, n, cols] and grad_y[t, cols], tokens 4q..4q+3
-  u32x4 gA[PreDims<N>::MK][2];        // grad_mixes row of token tb + r (A of gs), hi/lo
-  u32x2 ga[PreDims<N>::MT][2];        // (grad_mixes*inv)^T, tokens 4q..4q+3 (A of grad_phi)
-  float4 cf[4];                       // {pre[t,n], inv[t], scale[t]} of tokens 4q..4q+3
-};
+}  // namespace mhc
 
-template <int N, int P>
-__global__ __launch_bounds__(64 * N) void pre_bwd_stream_kernel(PreBwdStreamArgs a) {
-  using PD = PreDims<N>;
-  using Tile = StreamTile<N>;
-  typedef typename Tile::Row Row;
-  constexpr int M = PD::M, MT = PD::MT, MK = PD::MK, MP32 = PD::MP32;
-  constexpr int VC = StreamCfg<N>::VC, DW = StreamCfg<N>::DW, VD = VC / 2;
-  constexpr int TT = kStreamTile;
+#include "pre_bwd_gen.hpp"
 
-  const int lane = threadIdx.x & (kWave - 1);
-  const int n = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane & 15, q = lane >> 4;
-  const int D = a.D;
-  const int64_t K = (int64_t)N * D, T = a.T;
-  const int dl = blockIdx.x * DW + VC * r;  // first column d of this lane
-  const bool colok = dl < D;                // D % VC == 0 on this path
-  const int dlc = colok ? dl : 0;           // clamped column for branch-free loads
-  const int64_t kcol = (int64_t)n * D + dl;
-
-  u32x4 pb[VC][MK][P];
-#pragma unroll
-  for (int c = 0; c < VC; ++c)
-#pragma unroll
-    for (int mk = 0; mk < MK; ++mk)
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-        pb[c][mk][p] = colok ? ld16(a.phiT + p * a.phiT_plane_stride + (kcol + c) * MP32 + 32 * mk + 8 * q)
-                             : zero4();
-
-  floatx4 ph[MT][VC];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int c = 0; c < VC; ++c) ph[mt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  // Loads are unconditional from clamped addresses and their data is used
-  // unmodified, so a tile's loads issue back to back and stay in flight
-  // until compute_tile: a clamped x row meets zero columns of g (kernel A
-  // zero-fills the padding tokens of the last tile), clamped gm rows and
-  // coefficients only reach outputs of tokens >= T, which are not stored.
-  // With one phi plane the x / grad_y rows (HBM) are loaded one tile ahead,
-  // after the current tile's workspace operands (L2): vector loads complete
-  // in issue order, so waiting for those operands leaves the next rows in
-  // flight (N = 8, D = 2048: 1.49 -> 1.34 ms for the backward on MI355X).  A
-  // whole second tile of operands would not fit the 256 VGPRs of two waves
-  // per SIMD; with two phi planes even the rows spill (1.78 -> 2.14 ms), so
-  // that form loads a tile and then computes it.
-  auto load_rows = [&](int64_t tile, Row* xr, Row* gr) {
-    const int64_t tg = tile * TT + 4 * q;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t t = tg + e;
-      const int64_t tc = t < T ? t : T - 1;
-      xr[e] = __builtin_nontemporal_load(reinterpret_cast<const Row*>(a.x + (tc * N + n) * D + dlc));
-      gr[e] = *reinterpret_cast<const Row*>(a.gy + tc * D + dlc);
-    }
-  };
-  auto load_operands = [&](int64_t tile, Tile& tl) {
-    const int64_t tb = tile * TT, tg = tb + 4 * q;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t t = tg + e;
-      const int64_t tc = t < T ? t : T - 1;
-      tl.cf[e] = a.coef[tc * N + n];
-    }
-    const int64_t ts = tb + r;  // token of MFMA row r in the gs product
-    const int64_t tsc = ts < T ? ts : T - 1;
-#pragma unroll
-    for (int mk = 0; mk < MK; ++mk)
-#pragma unroll
-      for (int g = 0; g < 2; ++g) tl.gA[mk][g] = ld16(a.gmP + g * a.gmP_plane + tsc * MP32 + 32 * mk + 8 * q);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const u32x4 v = ld16(a.gTw + ((tile * MT + mt) * 64 + lane) * 8);
-      tl.ga[mt][0] = u32x2{v[0], v[1]};
-      tl.ga[mt][1] = u32x2{v[2], v[3]};
-    }
-  };
-
-  auto compute_tile = [&](int64_t tile, const Tile& tl) {
-    const int64_t tg = tile * TT + 4 * q;
-    // ---- grad_phi partial += g^T @ x over the tile's 16 tokens ----------
-#pragma unroll
-    for (int c = 0; c < VC; ++c) {
-      // column c of the lane's 4 x VC block: tokens (2w, 2w+1) in dword w
-      u32x2 xt;
-#pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        const uint32_t lo = tl.xr[2 * w][c >> 1], hi = tl.xr[2 * w + 1][c >> 1];
-        xt[w] = (c & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        ph[mt][c] = mfma16x16x16(tl.ga[mt][0], xt, ph[mt][c]);
-        ph[mt][c] = mfma16x16x16(tl.ga[mt][1], xt, ph[mt][c]);
-      }
-    }
-    // ---- gs = grad_mixes @ phi, then grad_x ---------------------------------
-    floatx4 gs[VC];
-#pragma unroll
-    for (int c = 0; c < VC; ++c) {
-      gs[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int mk = 0; mk < MK; ++mk) {
-        gs[c] = mfma16x16x32(as_bf16x8(tl.gA[mk][0]), as_bf16x8(pb[c][mk][0]), gs[c]);
-        gs[c] = mfma16x16x32(as_bf16x8(tl.gA[mk][1]), as_bf16x8(pb[c][mk][0]), gs[c]);
-        if constexpr (P > 1) gs[c] = mfma16x16x32(as_bf16x8(tl.gA[mk][0]), as_bf16x8(pb[c][mk][P - 1]), gs[c]);
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t t = tg + e;
-      if (!(colok && t < T)) continue;
-      const float4 cf = tl.cf[e];  // pre[t,n], inv[t], scale[t]
-      Row o;
-#pragma unroll
-      for (int w = 0; w < VD; ++w) {
-        const uint32_t xw = tl.xr[e][w], gw = tl.gr[e][w];
-        const float x0 = __uint_as_float(xw << 16), x1 = __uint_as_float(xw & 0xffff0000u);
-        const float g0 = __uint_as_float(gw << 16), g1 = __uint_as_float(gw & 0xffff0000u);
-        const float o0 = fmaf(cf.z, x0, fmaf(cf.y, gs[2 * w][e], g0 * cf.x));
-        const float o1 = fmaf(cf.z, x1, fmaf(cf.y, gs[2 * w + 1][e], g1 * cf.x));
-        o[w] = pack_bf16x2(o0, o1);
-      }
-      *reinterpret_cast<Row*>(a.gx + (t * N + n) * D + dl) = o;
-    }
-  };
-
-  const int64_t ntiles = (T + TT - 1) / TT;
-  if constexpr (P == 1) {
-    Row xn[4], gn[4];  // rows of the next tile
-    if (blockIdx.y < ntiles) load_rows(blockIdx.y, xn, gn);
-    for (int64_t tile = blockIdx.y; tile < ntiles; tile += a.nsplit) {
-      Tile A;
-      load_operands(tile, A);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        A.xr[e] = xn[e];
-        A.gr[e] = gn[e];
-      }
-      if (tile + a.nsplit < ntiles) load_rows(tile + a.nsplit, xn, gn);
-      compute_tile(tile, A);
-    }
-  } else {
-    for (int64_t tile = blockIdx.y; tile < ntiles; tile += a.nsplit) {
-      Tile A;
-      load_rows(tile, A.xr, A.gr);
-      load_operands(tile, A);
-      compute_tile(tile, A);
-    }
-  }
-
-  if (!colok) return;
-  float* part = a.gphi_part + (int64_t)blockIdx.y * M * K;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int m = 16 * mt + 4 * q + v;
-      if (m >= M) continue;
-#pragma unroll
-      for (int c = 0; c < VC; ++c) part[(int64_t)m * K + kcol + c] = ph[mt][c][v];
-    }
-}
+namespace mhc {
 
 // ---------------------------------------------------------------------------
 // Kernel B, LDS-pipelined form (N = 4 / 8, bf16 activations, 16-byte rows)
 //
-// Same per-lane arithmetic as the streaming form, but the operands of a
+// The per-lane arithmetic of the general kernel, but the operands of a
 // 16-token tile reach the lanes through a ring of S stages in LDS filled by
 // direct-to-LDS loads (buffer_load ... lds / global_load_lds): a tile's
 // loads are issued S-1 tiles before it is computed and cost no registers
@@ -1717,8 +1279,8 @@ __global__ void zero_kernel(float* p, int64_t n) {
 // host side
 // ---------------------------------------------------------------------------
 struct BwdLayout {
-  int M, L, C, P, MP, MP32, nsplit, chunks, DC, gpre_chunks;
-  int64_t K, nblkA, tok_per_split, ntiles;
+  int M, L, C, P, MP, MP32, gpre_chunks;
+  int64_t K, nblkA, ntiles;
   size_t off_phiT, off_gm, off_scale, off_partial, off_gphi, off_sink, off_gpre, off_gpl;
   size_t off_gmP, off_gTw, off_coef, total;
   // single-pass form (0 when it cannot apply): G members per group, control
@@ -1758,9 +1320,7 @@ static int64_t dma_max_splits(int D) {
   return s > kMaxSplits ? s : kMaxSplits;
 }
 
-// Workspace layout.  It covers both forms of kernel B (the streaming one for
-// bf16 activations and the LDS-staged one for the other dtypes / unaligned
-// rows), so the size depends only on (T, N, D, phi dtype, iterations).
+// Workspace layout.  It covers both forms of kernel B, so the size depends only on (T, N, D, phi dtype, iterations).
 static BwdLayout bwd_layout(int64_t T, int N, int D, int32_t phi_dtype, int iters) {
   BwdLayout b{};
   b.M = 2 * N + N * N;
@@ -1770,19 +1330,8 @@ static BwdLayout bwd_layout(int64_t T, int N, int D, int32_t phi_dtype, int iter
   b.MP = (int)round_up(b.M, 16);
   b.MP32 = (int)round_up(b.M, 32);
   b.K = (int64_t)N * D;
-  b.DC = kMainKC / N;
-  b.chunks = (int)((D + b.DC - 1) / b.DC);
   b.nblkA = (T + kBwdTile - 1) / kBwdTile;
   b.ntiles = (T + kStreamTile - 1) / kStreamTile;
-  int ns = (1024 + b.chunks - 1) / b.chunks;
-  if (ns > kMaxSplits) ns = kMaxSplits;
-  const int64_t max_by_t = (T + kMainTS - 1) / kMainTS;
-  if (ns > max_by_t) ns = (int)max_by_t;
-  if (ns < 1) ns = 1;
-  b.tok_per_split = round_up((T + ns - 1) / ns, kMainTS);
-  if (b.tok_per_split < kMainTS) b.tok_per_split = kMainTS;
-  b.nsplit = (int)((T + b.tok_per_split - 1) / b.tok_per_split);
-  if (b.nsplit < 1) b.nsplit = 1;
   size_t off = 0;
   b.off_phiT = off;
   off += align256(phiT_planes_bytes(phi_dtype, b.M, b.K));
@@ -1824,31 +1373,6 @@ static BwdLayout bwd_layout(int64_t T, int N, int D, int32_t phi_dtype, int iter
   if (b.bcG) off += align256((size_t)kCoCtlWords * 4) + align256(b.bc_ring_bytes);
   b.total = off;
   return b;
-}
-
-template <int N, int P>
-static int stream_blocks_per_cu() {
-  static std::atomic<int> cache{0};
-  int nb = cache.load(std::memory_order_relaxed);
-  if (nb > 0) return nb;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, pre_bwd_stream_kernel<N, P>, 64 * N, 0) != hipSuccess || nb <= 0)
-    nb = 1;
-  cache.store(nb, std::memory_order_relaxed);
-  return nb;
-}
-
-template <int N, int P>
-static int launch_stream(const BwdLayout& lay, PreBwdStreamArgs& sta, hipStream_t st) {
-  constexpr int DW = StreamCfg<N>::DW;
-  const int chunks = (int)((lay.K / N + DW - 1) / DW);
-  int64_t ns = (int64_t)device_cu_count() * stream_blocks_per_cu<N, P>() / chunks;
-  if (ns > kMaxSplits) ns = kMaxSplits;
-  if (ns > lay.ntiles) ns = lay.ntiles;
-  if (ns < 1) ns = 1;
-  sta.nsplit = (int)ns;
-  hipLaunchKernelGGL((pre_bwd_stream_kernel<N, P>), dim3((unsigned)chunks, (unsigned)ns),
-                     dim3(64 * N), 0, st, sta);
-  return check_launch("pre_bwd_stream");
 }
 
 static unsigned reduce_grid(int64_t n) {
@@ -1940,16 +1464,16 @@ static int launch_dma(const BwdLayout& lay, const PreBwdStreamArgs& sta, int* ns
   if (ns > lay.ntiles) ns = lay.ntiles;
   if (ns < 1) ns = 1;
   PreBwdDmaArgs da{};
-  da.x = sta.x;
-  da.gy = sta.gy;
+  da.x = static_cast<const bf16_t*>(sta.x);
+  da.gy = static_cast<const bf16_t*>(sta.gy);
   da.phiT = sta.phiT;
   da.phiT_plane_stride = sta.phiT_plane_stride;
   da.gmP = sta.gmP;
   da.gmP_plane = sta.gmP_plane;
   da.gTw = sta.gTw;
   da.coef = sta.coef;
-  da.gx = sta.gx;
-  da.gin = sta.gin;
+  da.gx = static_cast<bf16_t*>(sta.gx);
+  da.gin = static_cast<const bf16_t*>(sta.gin);
   da.part = sta.gphi_part;
   da.T = sta.T;
   da.D = D;
@@ -1968,18 +1492,28 @@ static int launch_dma(const BwdLayout& lay, const PreBwdStreamArgs& sta, int* ns
   return check_launch("pre_bwd_dma");
 }
 
-// grad_x += grad_x_in for the kernels without an accumulating form
-template <typename S>
-__global__ void add_into_kernel(S* out, const S* in, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    store_elem(out, i, load_elem(out, i) + load_elem(in, i));
-}
-
-template <typename S>
-static int add_into(void* out, const void* in, int64_t n, hipStream_t st) {
-  hipLaunchKernelGGL((add_into_kernel<S>), dim3(reduce_grid(n)), dim3(256), 0, st, static_cast<S*>(out),
-                     static_cast<const S*>(in), n);
-  return check_launch("pre_bwd_add_into");
+// The general kernel B; *nsplit receives its token-split count: as many as
+// give every CU two blocks (N = 8: one), at least four tiles a block where
+// that still leaves a block for every CU (each split's partials are written
+// and read once: 8 * M bytes a column against 32 * sizeof(S) a tile of x).
+template <int N, typename S, int P>
+static int launch_gen_bwd(const BwdLayout& lay, const PreBwdStreamArgs& sta, int* nsplit, hipStream_t st) {
+  using C = GenBwdCfg<N, S>;
+  // a wave's columns: a stream's, cut at multiples of VC (up to VC - 1 more)
+  const int64_t most = sta.D % C::VC ? sta.D + C::VC - 1 : sta.D;
+  const int64_t ncb = (most + C::DW - 1) / C::DW * C::NG, cus = device_cu_count();
+  int64_t ns = C::BLOCKS_PER_CU * cus / ncb;
+  if (ns > lay.ntiles / 4) ns = lay.ntiles / 4 > cus / ncb ? lay.ntiles / 4 : cus / ncb;
+  if (ns > dma_max_splits(sta.D)) ns = dma_max_splits(sta.D);
+  if (ns > lay.ntiles) ns = lay.ntiles;
+  if (ns < 1) ns = 1;
+  const dim3 grid((unsigned)ncb, (unsigned)ns);
+  if (sta.D % C::VC)
+    hipLaunchKernelGGL((pre_bwd_gen_kernel<N, S, P, true>), grid, dim3(C::THREADS), 0, st, sta, lay.ntiles);
+  else
+    hipLaunchKernelGGL((pre_bwd_gen_kernel<N, S, P, false>), grid, dim3(C::THREADS), 0, st, sta, lay.ntiles);
+  *nsplit = (int)ns;
+  return check_launch("pre_bwd_gen");
 }
 
 // The single-pass form (pre_bwd_coop.hpp) where it applies: kernel A's SP
@@ -2010,13 +1544,13 @@ static int launch_pre_bwd_coop(const BwdLayout& lay, PreBwdSmallArgs sa, const P
   sa.scale = nullptr;
   sa.gpre_part = nullptr;
   sa.coefX = reinterpret_cast<float*>(ws + lay.off_coef);
-  hipLaunchKernelGGL((pre_bwd_small_kernel<4, bf16_t, true, true>), dim3((unsigned)lay.nblkA), dim3(kBwdThreads), 0,
+  hipLaunchKernelGGL((pre_bwd_small_kernel<4, bf16_t, true>), dim3((unsigned)lay.nblkA), dim3(kBwdThreads), 0,
                      st, sa);
   if ((rc = check_launch("pre_bwd_small_sp"))) return rc;
   BwdCoopArgs ca{};
-  ca.x = sta.x;
-  ca.gy = sta.gy;
-  ca.gx = sta.gx;
+  ca.x = static_cast<const bf16_t*>(sta.x);
+  ca.gy = static_cast<const bf16_t*>(sta.gy);
+  ca.gx = static_cast<bf16_t*>(sta.gx);
   ca.phiT = sta.phiT;
   ca.gm = sa.gm;
   ca.coefX = sa.coefX;
@@ -2034,16 +1568,15 @@ static int launch_pre_bwd_coop(const BwdLayout& lay, PreBwdSmallArgs sa, const P
   if ((rc = check_launch("pre_bwd_coop"))) return rc;
   *used = true;
   const int64_t n = (int64_t)lay.M * lay.K;
-  hipLaunchKernelGGL(bc_sum_kernel, dim3(reduce_grid(n)), dim3(256), 0, st, sta.gphi_part, grad_phi, n, ctl, sta.gx,
+  hipLaunchKernelGGL(bc_sum_kernel, dim3(reduce_grid(n)), dim3(256), 0, st, sta.gphi_part, grad_phi, n, ctl, ca.gx,
                      sa.T * lay.K, status_out);
   if ((rc = check_launch("pre_bwd_coop_sum"))) return rc;
   return sum_alpha_base(lay, sa, grad_alpha, grad_base, st, lay.bc_rows, ctl + kCtlStatus);
 }
 
 template <int N, typename S>
-static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwdMainArgs& ma,
-                          PreBwdStreamArgs sta, float* grad_phi, float* grad_alpha,
-                          float* grad_base, bool vec, const void* gin, uint16_t* gpl, hipStream_t st,
+static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwdStreamArgs& sta, float* grad_phi,
+                          float* grad_alpha, float* grad_base, bool vec, const void* gin, uint16_t* gpl, hipStream_t st,
                           char* ws, int sp_mode, int32_t* status_out) {
   const dim3 gA((unsigned)lay.nblkA), bA(kBwdThreads);
   const bool streaming = vec && std::is_same<S, bf16_t>::value;
@@ -2057,14 +1590,8 @@ static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwd
       if (rc || used) return rc;
     }
   }
-  if (streaming) {
-    if (!sa.comp) sa.gm = nullptr;  // the compensated grad_phi reads fp32 grad_mixes
-    sa.scale = nullptr;
-  } else {
-    sa.gmP = nullptr;
-    sa.gTw = nullptr;
-    sa.coef = nullptr;
-  }
+  if (!sa.comp) sa.gm = nullptr;  // only the compensated grad_phi reads fp32 grad_mixes
+  sa.scale = nullptr;
   int rc;
   if (streaming && sa.T >= kGpreDmaMinT) {
     // grad_pre through the LDS-pipelined kernel: one chunk of sums per token
@@ -2077,54 +1604,32 @@ static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwd
   } else if (sa.gpre_part) {
     const dim3 gG((unsigned)(sa.T < kGpreGridT ? sa.T : kGpreGridT), (unsigned)lay.gpre_chunks);
     float* part = const_cast<float*>(sa.gpre_part);
-    if (vec)
-      hipLaunchKernelGGL((pre_bwd_gpre_kernel<N, S, true>), gG, bA, 0, st, sa.x, sa.gy, part, sa.T, sa.D);
-    else
-      hipLaunchKernelGGL((pre_bwd_gpre_kernel<N, S, false>), gG, bA, 0, st, sa.x, sa.gy, part, sa.T, sa.D);
+    hipLaunchKernelGGL((pre_bwd_gpre_kernel<N, S>), gG, bA, 0, st, sa.x, sa.gy, part, sa.T, sa.D);
     if ((rc = check_launch("pre_bwd_gpre"))) return rc;
   }
-  if (vec)
-    hipLaunchKernelGGL((pre_bwd_small_kernel<N, S, true>), gA, bA, 0, st, sa);
-  else
-    hipLaunchKernelGGL((pre_bwd_small_kernel<N, S, false>), gA, bA, 0, st, sa);
+  hipLaunchKernelGGL((pre_bwd_small_kernel<N, S>), gA, bA, 0, st, sa);
   rc = check_launch("pre_bwd_small");
   if (rc) return rc;
-  if (streaming && dma_usable<N>(sta.D)) {
-    sta.gin = static_cast<const bf16_t*>(gin);  // accumulated inside the kernel
-    int ns = 0;
+  int ns = 0;
+  if (streaming && dma_usable<N>(sta.D))
     rc = lay.P == 1 ? launch_dma<N, 1>(lay, sta, &ns, st) : launch_dma<N, 2>(lay, sta, &ns, st);
-    if (rc) return rc;
-    return reduce_tail<N, S>(lay, sa, sta.gphi_part, ns, gpl, grad_phi, grad_alpha, grad_base, st);
-  }
-  const int64_t nx = sta.T * N * (int64_t)sta.D;
-  if (streaming) {
-    rc = lay.P == 1 ? launch_stream<N, 1>(lay, sta, st) : launch_stream<N, 2>(lay, sta, st);
-    if (rc) return rc;
-    if (gin && (rc = add_into<S>(sta.gx, gin, nx, st))) return rc;
-    return reduce_tail<N, S>(lay, sa, sta.gphi_part, sta.nsplit, gpl, grad_phi, grad_alpha, grad_base, st);
-  }
-  const dim3 gB((unsigned)lay.chunks, (unsigned)lay.nsplit), bB(256);
-  if (vec)
-    hipLaunchKernelGGL((pre_bwd_main_kernel<N, S, true>), gB, bB, 0, st, ma);
   else
-    hipLaunchKernelGGL((pre_bwd_main_kernel<N, S, false>), gB, bB, 0, st, ma);
-  rc = check_launch("pre_bwd_main");
+    rc = lay.P == 1 ? launch_gen_bwd<N, S, 1>(lay, sta, &ns, st) : launch_gen_bwd<N, S, 2>(lay, sta, &ns, st);
   if (rc) return rc;
-  if (gin && (rc = add_into<S>(ma.gx, gin, nx, st))) return rc;
-  return reduce_tail<N, S>(lay, sa, ma.gphi_part, lay.nsplit, gpl, grad_phi, grad_alpha, grad_base, st);
+  return reduce_tail<N, S>(lay, sa, sta.gphi_part, ns, gpl, grad_phi, grad_alpha, grad_base, st);
 }
 
 template <typename S>
 static int dispatch_pre_bwd(int N, const BwdLayout& lay, const PreBwdSmallArgs& sa,
-                            const PreBwdMainArgs& ma, const PreBwdStreamArgs& sta, float* gphi,
+                            const PreBwdStreamArgs& sta, float* gphi,
                             float* galpha, float* gbase, bool vec, const void* gin, uint16_t* gpl,
                             hipStream_t st, char* ws, int sp_mode, int32_t* status_out) {
   switch (N) {
     case 4:
-      return launch_pre_bwd<4, S>(lay, sa, ma, sta, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
+      return launch_pre_bwd<4, S>(lay, sa, sta, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
                                   status_out);
     case 8:
-      return launch_pre_bwd<8, S>(lay, sa, ma, sta, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
+      return launch_pre_bwd<8, S>(lay, sa, sta, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
                                   status_out);
   }
   return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_bwd: N=%d not supported (4, 8)", N);
@@ -2209,34 +1714,18 @@ static int pre_bwd_entry(const void* x, int32_t x_dtype, const void* phi, int32_
   sa.T = T;
   sa.D = D;
 
-  PreBwdMainArgs ma{};
-  ma.x = x;
-  ma.gy = grad_y;
-  ma.phiT = phiT;
-  ma.phiT_plane_stride = lay.K * lay.MP32;
-  ma.phi_planes = lay.P;
-  ma.gm = sa.gm;
-  ma.inv_rms = inv_rms;
-  ma.pre = pre;
-  ma.scale = sa.scale;
-  ma.gx = grad_x;
-  ma.gphi_part = reinterpret_cast<float*>(ws + lay.off_gphi);
-  ma.T = T;
-  ma.D = D;
-  ma.tok_per_split = lay.tok_per_split;
-
   PreBwdStreamArgs sta{};
-  sta.x = static_cast<const bf16_t*>(x);
-  sta.gy = static_cast<const bf16_t*>(grad_y);
+  sta.x = x;
+  sta.gy = grad_y;
+  sta.gin = grad_x_in;
   sta.phiT = phiT;
   sta.phiT_plane_stride = lay.K * lay.MP32;
-  sta.phi_planes = lay.P;
   sta.gmP = sa.gmP;
   sta.gmP_plane = sa.gmP_plane;
   sta.gTw = sa.gTw;
   sta.coef = sa.coef;
-  sta.gx = static_cast<bf16_t*>(grad_x);
-  sta.gphi_part = ma.gphi_part;
+  sta.gx = grad_x;
+  sta.gphi_part = reinterpret_cast<float*>(ws + lay.off_gphi);
   sta.T = T;
   sta.D = D;
 
@@ -2246,13 +1735,13 @@ static int pre_bwd_entry(const void* x, int32_t x_dtype, const void* phi, int32_
   const int sp = (flags & MHC_PRE_BWD_TWO_PASS) ? 0 : (flags & MHC_PRE_BWD_SINGLE_PASS) ? 2 : 1;
   switch (x_dtype) {
     case MHC_DTYPE_BF16:
-      return dispatch_pre_bwd<bf16_t>(N, lay, sa, ma, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
+      return dispatch_pre_bwd<bf16_t>(N, lay, sa, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
                                       ws, sp, status);
     case MHC_DTYPE_F16:
-      return dispatch_pre_bwd<f16_t>(N, lay, sa, ma, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
+      return dispatch_pre_bwd<f16_t>(N, lay, sa, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
                                      ws, sp, status);
     case MHC_DTYPE_F32:
-      return dispatch_pre_bwd<float>(N, lay, sa, ma, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
+      return dispatch_pre_bwd<float>(N, lay, sa, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
                                      ws, sp, status);
   }
   return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_bwd: x dtype %d not supported", x_dtype);

@@ -174,4 +174,49 @@ __device__ __forceinline__ void load8f(const S* p, int64_t k, int64_t lim, bool 
   }
 }
 
+// Eight consecutive elements as loaded.
+template <typename S> struct Raw8 { u32x4 v[sizeof(S) / 2]; };
+
+// Global loads and stores of rows at any element alignment: unaligned 16- and
+// 8-byte accesses are single instructions on this part.
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 ld16u(const void* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
+
+template <typename S>
+__device__ __forceinline__ Raw8<S> gen_load8(const S* p) {
+  Raw8<S> r;
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(S) / 2; ++i) r.v[i] = ld16u(reinterpret_cast<const char*>(p) + 16 * i);
+  return r;
+}
+// elements [k, k + 8) of a row of `lim`: those past it are zero
+template <typename S>
+__device__ __forceinline__ Raw8<S> gen_load8_tail(const S* row, int64_t k, int64_t lim) {
+  Raw8<S> r;
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(S) / 2; ++i) r.v[i] = zero4();
+  if constexpr (sizeof(S) == 2) {
+    const uint16_t* p = reinterpret_cast<const uint16_t*>(row);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (k + i < lim) r.v[0][i / 2] |= (uint32_t)p[k + i] << (16 * (i & 1));
+  } else {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(row);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (k + i < lim) r.v[i / 4][i & 3] = p[k + i];
+  }
+  return r;
+}
+
+// Eight elements [k, k + 8) of a row of `lim` as fp32, any alignment; zero
+// past the row.
+template <typename S>
+__device__ __forceinline__ void load8u(const S* row, int64_t k, int64_t lim, float* f) {
+  const Raw8<S> r = k + 8 <= lim ? gen_load8(row + k) : gen_load8_tail(row, k, lim);
+  Store<S>::unpack(r.v[0], f);
+  if constexpr (sizeof(S) == 4) Store<S>::unpack(r.v[1], f + 4);
+}
+
 }  // namespace mhc

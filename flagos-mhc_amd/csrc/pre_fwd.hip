@@ -1244,7 +1244,7 @@ static size_t pre_fwd_ws_min(int64_t T, int32_t N, int32_t D, int32_t phi_dtype)
 extern "C" size_t mhc_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, int32_t phi_dtype) {
   size_t base = pre_fwd_ws_min(T, N, D, phi_dtype);
   if (N != 4 && N != 8) return base;
-  if (phi_dtype != MHC_DTYPE_BF16 || (int64_t)N * D % 8) {  // the general form's sums
+  if (phi_dtype != MHC_DTYPE_BF16 || D % 8) {  // the general form's sums
     const size_t gen = D > 0 && T > 0 ? gen_ws_bytes(T, N, D) : 0;
     return gen > base ? gen : base;
   }

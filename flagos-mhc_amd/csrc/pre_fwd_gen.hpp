@@ -65,38 +65,6 @@ template <int N, bool SMALL> struct GenCfg {
   __device__ static constexpr int swz(int row) { return CW == 64 ? ((row >> 1) & 7) : (row & 15); }
 };
 
-// Eight consecutive elements as loaded.
-template <typename S> struct Raw8 { u32x4 v[sizeof(S) / 2]; };
-
-typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
-__device__ __forceinline__ u32x4 ld16u(const void* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
-
-template <typename S>
-__device__ __forceinline__ Raw8<S> gen_load8(const S* p) {
-  Raw8<S> r;
-#pragma unroll
-  for (int i = 0; i < (int)sizeof(S) / 2; ++i) r.v[i] = ld16u(reinterpret_cast<const char*>(p) + 16 * i);
-  return r;
-}
-// elements [k, k + 8) of a row of `lim`: those past it are zero
-template <typename S>
-__device__ __forceinline__ Raw8<S> gen_load8_tail(const S* row, int64_t k, int64_t lim) {
-  Raw8<S> r;
-#pragma unroll
-  for (int i = 0; i < (int)sizeof(S) / 2; ++i) r.v[i] = zero4();
-  if constexpr (sizeof(S) == 2) {
-    const uint16_t* p = reinterpret_cast<const uint16_t*>(row);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (k + i < lim) r.v[0][i / 2] |= (uint32_t)p[k + i] << (16 * (i & 1));
-  } else {
-    const uint32_t* p = reinterpret_cast<const uint32_t*>(row);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (k + i < lim) r.v[i / 4][i & 3] = p[k + i];
-  }
-  return r;
-}
 template <typename S>
 __device__ __forceinline__ void gen_unpack(const Raw8<S>& r, float (&f)[8]) {
   if constexpr (sizeof(S) == 2) {
@@ -122,7 +90,6 @@ __device__ __forceinline__ void gen_planes(const Raw8<S>& r, const float (&f)[8]
 // every 16-byte access of a wave continues its neighbour's (4-byte elements
 // stored as 16-byte pieces at a 32-byte lane stride move at a third of the
 // rate).
-typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 template <typename S, bool SPLIT>
 __device__ __forceinline__ Raw8<S> gen_load_chunk(const S* row, int c0, int lane, int lim) {
   if constexpr (!SPLIT) {

@@ -106,10 +106,11 @@ int mhc_post_bwd_sum_fused(int64_t T, int32_t N, int32_t D, int32_t dtype);
  * x and phi, D = 4096 or 7168 .. 8192 and T >= 8192, the exchange ring of the
  * single-pass form (x read from HBM once, ~13 MB + 120 bytes per token); a
  * smaller workspace that still holds the two-pass forms' runs those.  For phi
- * that is not bf16 (or whose rows are no multiple of 16 bytes) it includes the
+ * that is not bf16, or D % 8 != 0, it includes the
  * general form's sums over split columns (at most ~128 * 25 floats a token at
  * few tokens, ~3 * 25 from 16384 on); with less, the tokens run in chunks that
- * fit, or in a slower form that needs only phi's bf16 planes.
+ * fit, or in a slower form that needs only phi's bf16 planes.  x that is not
+ * bf16 runs the general form whatever phi is: ask with MHC_DTYPE_F32 then.
  */
 size_t mhc_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, int32_t phi_dtype);
 int mhc_pre_fwd(const void* x, int32_t x_dtype, const void* phi, int32_t phi_dtype,
