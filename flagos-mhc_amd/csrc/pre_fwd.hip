@@ -1136,6 +1136,7 @@ static int launch_pre_fwd_dma(PreFwdArgs a, void* workspace, size_t workspace_by
                        dim3(kFwdThreads), 0, st, a);
     int rc = check_launch("pre_fwd_split");
     if (rc) return rc;
+    if (finish_applies(a.T, N, a.D)) return launch_pre_fwd_finish<N, bf16_t>(a, plan.nsplit, st);
     constexpr int TPP = kFwdThreads / (N * N);
     hipLaunchKernelGGL((pre_fwd_finalize_kernel<N>), dim3((unsigned)((a.T + TPP - 1) / TPP)), dim3(kFwdThreads),
                        0, st, a, plan.nsplit);
@@ -1169,6 +1170,7 @@ static int launch_pre_fwd_dma(PreFwdArgs a, void* workspace, size_t workspace_by
   int rc = check_launch("pre_fwd_dma");
   if (rc) return rc;
   if constexpr (FwdDmaCfg<N>::HEADS_APART) {
+    if (finish_applies(a.T, N, a.D)) return launch_pre_fwd_finish<N, bf16_t>(a, 1, st);
     constexpr int TPP = kFwdThreads / (N * N);
     hipLaunchKernelGGL((pre_fwd_finalize_kernel<N>), dim3((unsigned)((a.T + TPP - 1) / TPP)), dim3(kFwdThreads),
                        0, st, a, 1);

@@ -396,7 +396,8 @@ __device__ __forceinline__ void gen_y8(const PreFwdArgs& a, int64_t t, int c0, i
   gen_store_chunk<S, kGenSplit<S, XS>>(static_cast<S*>(a.y) + t * D, c0, lane, D, o);
 }
 
-// One block per token (few tokens: the time is latency).  All waves add the
+// One block per token, after the general contraction or the LDS-pipelined
+// kernels' sums (see finish_applies).  All waves add the
 // slots, wave 0 then runs the heads and Sinkhorn while the others form y from
 // rows they began to load before the sums were complete; y needs only the
 // pre gates, which every wave forms for itself.
@@ -467,7 +468,36 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_finish_kernel(Pr
   if (ok) a.comb[t * L + e] = c;
 }
 
+// y (and x_scaled) after the finalize kernel: a block per token of W waves,
+// wave w taking the 512-column chunks w, w + W, ..
+template <int N, typename S, bool XS>
+__global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_gen_y_kernel(PreFwdArgs a) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = blockDim.x / kWave;
+  const int64_t t = blockIdx.x;
+  float p[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) p[n] = a.pre_ws[t * N + n];
+  const float inv = XS ? a.inv_ws[t] : 0.f;
+  for (int c0 = wave * 512; c0 < a.D; c0 += W * 512) {
+    Raw8<S> X[N];
+    gen_load_rows<N, S, XS>(a, t, c0, lane, X);
+    gen_y8<N, S, XS>(a, t, c0, lane, X, p, inv);
+  }
+}
+
 // ---- host side --------------------------------------------------------------
+// Whether the finish kernel ends a call, rather than the finalize kernel
+// (tokens packed N * N lanes each) and a y kernel.  Its Sinkhorn wave per token
+// hides behind the token's y only where that is long enough, or where so few
+// tokens run that a launch less is what counts.  Measured (bf16, us, finish /
+// finalize + y, whole operator): N = 4: D = 256 T = 2048 14.2 / 13.0, T =
+// 16384 39.9 / 25.8; D = 512 T = 4096 16.5 / 17.6, T = 16384 41.9 / 37.9; D =
+// 1024 T = 16384 66.6 / 67.4; D = 5120 257 / 265; T = 64 D = 7168 11.6 / 16.1.
+// N = 8: D = 256 T = 16384 78.2 / 59.5; D = 512 78.3 / 86.3; D = 2048 T =
+// 32768 417 / 430.
+static bool finish_applies(int64_t T, int N, int D) { return T <= 1024 || D >= (N == 8 ? 512 : T <= 4096 ? 512 : 1024); }
+
 constexpr int kGenSmallT = 64;   // tokens up to which the 16-token tiles run
 constexpr int kGenFewUnits = 128;  // .. and stages of 128-token tiles below which they do
 constexpr int kGenMaxSlots = 128;  // slots of a tile's sums, at most about
@@ -541,7 +571,19 @@ static int launch_pre_fwd_gen_chunk(PreFwdArgs a, int32_t phi_dtype, char* w, hi
            : phi_dtype == MHC_DTYPE_F16 ? launch_gen_contraction<N, S, f16_t>(a, p, st)
                                         : launch_gen_contraction<N, S, float>(a, p, st);
   if (rc) return rc;
-  return launch_pre_fwd_finish<N, S>(a, 0, st);
+  if (finish_applies(a.T, N, a.D)) return launch_pre_fwd_finish<N, S>(a, 0, st);
+  constexpr int TPP = kFwdThreads / (N * N);
+  hipLaunchKernelGGL((pre_fwd_finalize_kernel<N>), dim3((unsigned)((a.T + TPP - 1) / TPP)), dim3(kFwdThreads), 0, st,
+                     a, 0);
+  if ((rc = check_launch("pre_fwd_finalize"))) return rc;
+  const int chunks = (a.D + 511) / 512;
+  const dim3 grid((unsigned)a.T), block(kWave * (chunks < kFinishWaves ? chunks : kFinishWaves));
+  if ((rc = check_grid(grid, block, "mhc_pre_fwd"))) return rc;
+  if (a.x_scaled)
+    hipLaunchKernelGGL((pre_fwd_gen_y_kernel<N, S, true>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((pre_fwd_gen_y_kernel<N, S, false>), grid, block, 0, st, a);
+  return check_launch("pre_fwd_gen_y");
 }
 
 // Tokens a call of the general form takes at a time in `bytes` of workspace:
