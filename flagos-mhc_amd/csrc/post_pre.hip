@@ -14,9 +14,18 @@
 // shape.  Where the pre forward has its single pass (T >= 8192, D = 4096 or
 // 7168 .. 8192) the single-pass pre kernel runs with a post front end
 // instead (post_pre_fwd_single_pass: x_next formed in the kernel, written
-// once, never read back), or, if that form cannot run, post then pre.  (The tile's gates sit in one LDS buffer that wave 0 refills when it
-// issues the next tile's first stage, S - 1 stages ahead: a tile must span
-// at least S stages, D >= 64 * S, so that it has read its gates by then.)
+// once, never read back), or, if that form cannot run, post then pre.
+//
+// Work split.  One block a CU takes whole tiles of 32 tokens in rounds; the
+// tiles left after the last full round are cut into runs of equal length, one
+// a block, whose sums go to slots in memory that the pre forward's finish (or
+// finalize) kernel adds (post_pre_plan).  With T a multiple of a round nothing
+// is left over and the kernel runs the heads itself (HEADS), hidden by the
+// next tile's loads.  Measured (bf16, us, whole operator, a tile a block as
+// before / now; MI355X): D = 7168: T = 64 152 / 15, T = 1024 168 / 50, T = 4096
+// 222 / 165, T = 9000 461 / 345, T = 8192 312 / 312; D = 5120, T = 5999 182 /
+// 172.  (A tile's gates sit in one of two LDS buffers; with D >= 64 S a buffer
+// is free again before the tile after the next one is loaded.)
 //
 // A block (8 waves, two per SIMD so that one wave's waits overlap the other's
 // work) owns a tile of 32 tokens.  Wave w handles row block rb = w & 1
@@ -39,9 +48,9 @@
 // each write 8 whole 128-byte row segments: lanes r and r ^ 8 trade their
 // second halves through a DPP row rotation first.  The four waves of a row
 // block hold partial sums over their streams; they are added in a fixed order
-// through LDS after the tile's last contraction stage, followed by heads and
-// Sinkhorn exactly as in the pre kernel; pre goes to the workspace for the y
-// kernel.  The y pass used to run as stages of this kernel (8 tokens x 4
+// through LDS after the tile's (or the run's) last contraction stage, followed
+// by heads and Sinkhorn as in the pre kernel, or stored; pre goes to the
+// workspace for the y kernel.  The y pass used to run as stages of this kernel (8 tokens x 4
 // streams x 512 columns each, which needed D >= 3136 so that a y stage's
 // loads followed the stores of its columns); as the block-per-token kernel
 // it is faster (N = 4, D = 7168, T = 65536: 2.55 -> 2.26 ms for the fused
@@ -76,13 +85,13 @@ struct PostPreArgs {
   const bf16_t* h_out;   // (T, D)
   const float* h_post;   // (T, 4)
   const uint16_t* phi;   // (M, 4D) bf16
+  bf16_t* x_next;        // (T, 4, D)
+  // HEADS: the pre operator's parameters and outputs but y
   const float* alpha;
   const float* base;
   float norm_eps, hc_eps, cmin, cmax;
   int apply_clamp;
   int iters;
-  bf16_t* x_next;        // (T, 4, D)
-  bf16_t* y;             // (T, D)
   float* post_out;
   float* comb;
   float* inv_rms;
@@ -90,6 +99,11 @@ struct PostPreArgs {
   float* logits;
   float* pre;
   float* pre_ws;         // (T, 4) pre for the y kernel
+  // otherwise
+  float* part;           // [slot][T][M] sums of x_next . phi^T over a run's columns of the tile
+  float* part_ssq;       // [slot][T] .. and of x_next^2
+  int64_t w;             // stages of a block's run
+  int rounds;            // whole tiles of every block before its run
   int64_t T;
   int D;
 };
@@ -100,6 +114,10 @@ __device__ __forceinline__ u32x4 lds_read1(uint32_t a) {
   return v;
 }
 
+// HEADS: every block takes whole tiles only and ends each with its heads and
+// Sinkhorn, which the next tile's loads hide (T a multiple of 32 tokens a CU);
+// otherwise the sums go to memory for the finish or finalize kernel.
+template <bool HEADS>
 __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a) {
   constexpr int N = kPPN, M = kPPM, MT = kPPMT, L = N * N, TT = kPPTile, S = kPPStages;
   // Stage j's loads have landed once at most V newer vector memory
@@ -111,9 +129,9 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
   constexpr int VM_C = (S - 2) * kPPCImin + (S - 1) * kPPCST;
   static_assert(VM_C < 64, "vmcnt range");
   __shared__ u32x4 ring[S * kPPUnits * kWave];
-  __shared__ u32x4 gates[3 * kWave];  // h_res rows of the 32 tokens (2 units), h_post (1 unit)
+  __shared__ u32x4 gates[2][3 * kWave];  // by tile parity: h_res rows of the 32 tokens (2 units), h_post (1 unit)
   __shared__ float red_ssq[2][3][16];
-  __shared__ float mix_sh[TT][M + 1];
+  __shared__ float mix_sh[HEADS ? TT : 1][M + 1];
   __shared__ __align__(16) float inv_sh[TT];
 
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -124,19 +142,50 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
   const int D = a.D;
   const int64_t K = (int64_t)N * D;
   const int64_t T = a.T;
-  const int nst_c = D / kPPCW;
-  const int per_tile = nst_c;
+  const int nst = D / kPPCW;
   const int64_t ntiles = (T + TT - 1) / TT;
-  const int64_t my_tiles = (ntiles - blockIdx.x + gridDim.x - 1) / gridDim.x;
-  if (my_tiles <= 0) return;  // uniform over the block
-  const int64_t J = my_tiles * per_tile;
+  // whole tiles b, b + blocks, .. in `rounds` rounds, then the block's run of
+  // the stages of the tiles left
+  const int rounds = a.rounds;
+  const int64_t left0 = (int64_t)rounds * gridDim.x, total = (ntiles - left0) * nst;
+  const int64_t u0 = (int64_t)blockIdx.x * a.w;
+  const int64_t run = u0 >= total ? 0 : (u0 + a.w < total ? a.w : total - u0);
+  const int64_t J = (int64_t)rounds * nst + run;
+  if (J <= 0) return;  // uniform over the block
+  struct Cursor {
+    int64_t tile;
+    int s, round, par;  // stage, tiles behind, gates buffer
+    bool fresh;         // the first stage of a tile in this block
+  };
+  auto start = [&]() {
+    Cursor c{rounds ? (int64_t)blockIdx.x : left0 + u0 / nst, rounds ? 0 : (int)(u0 % nst), 0, 0, true};
+    return c;
+  };
+  auto advance = [&](Cursor& c) {
+    c.fresh = false;
+    if (++c.s < nst) return;
+    c.s = 0;
+    c.par ^= 1;
+    c.fresh = true;
+    if (++c.round == rounds) {
+      c.tile = left0 + u0 / nst;
+      c.s = (int)(u0 % nst);
+    } else {
+      c.tile += c.round < rounds ? (int64_t)gridDim.x : 1;
+    }
+  };
   const auto rphi = rows_rsrc(a.phi, (int64_t)M * K * 2);
   const uint32_t gates_lds = lds_addr(gates);
 
   const int e = tid % L;
-  const float a0 = a.alpha[0], a1 = a.alpha[1], a2 = a.alpha[2];
-  const float base_l = a.base[2 * N + e];
-  const float base_h = e < 2 * N ? a.base[e] : 0.f;
+  float a0 = 0.f, a1 = 0.f, a2 = 0.f, base_l = 0.f, base_h = 0.f;
+  if constexpr (HEADS) {
+    a0 = a.alpha[0];
+    a1 = a.alpha[1];
+    a2 = a.alpha[2];
+    base_l = a.base[2 * N + e];
+    base_h = e < 2 * N ? a.base[e] : 0.f;
+  }
 
   // Per-lane byte offsets of this wave's contraction-stage units (u = wave +
   // 8i) at d0 = 0 (a stage adds 2*d0) and of its x_next stores; rows >= M of
@@ -179,25 +228,25 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
   }
 
   // ---- loads of stage j (issued S - 1 stages ahead) ------------------------
-  int64_t itile = blockIdx.x;
-  int is = 0;  // stage of the next issue
+  Cursor ic = start();
   auto issue = [&](int64_t j) {
-    const int64_t tb = itile * TT;
+    const int64_t tb = ic.tile * TT;
     const int nv = (int)(T - tb < TT ? T - tb : TT);
     const uint32_t slot = lds_addr(ring) + (uint32_t)((j % S) * kPPUnits * 1024);
-    if (is == 0 && wave == 0) {
+    if (ic.fresh && wave == 0) {
+      const uint32_t gl = gates_lds + (uint32_t)ic.par * (3 * kWave * 16);
       // the tile's gates: h_res rows (64 bytes a token), h_post (16 bytes)
       const auto rg = rows_rsrc(a.h_res + tb * L, (int64_t)nv * L * 4);
 #pragma unroll
       for (int u = 0; u < 2; ++u)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (lds_void_t*)(uintptr_t)(gates_lds + u * 1024), 16,
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rg, (lds_void_t*)(uintptr_t)(gl + u * 1024), 16,
                                                  (uint32_t)((16 * u + (lane >> 2)) * 64 + (lane & 3) * 16), 0,
                                                  0, 0);
       const auto rp = rows_rsrc(a.h_post + tb * N, (int64_t)nv * N * 4);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_void_t*)(uintptr_t)(gates_lds + 2048), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_void_t*)(uintptr_t)(gl + 2048), 16,
                                                lane < TT ? (uint32_t)(lane * 16) : kBufferOob, 0, 0, 0);
     }
-    const uint32_t d2 = (uint32_t)(is * kPPCW * 2);
+    const uint32_t d2 = (uint32_t)(ic.s * kPPCW * 2);
     const auto rx = rows_rsrc(a.x + tb * K, (int64_t)nv * K * 2);
     const auto rh = rows_rsrc(a.h_out + tb * D, (int64_t)nv * D * 2);
 #pragma unroll
@@ -213,10 +262,7 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rphi, dst, 16, cbase[i] + d2, 0, 0, 0);
       }
     }
-    if (++is == per_tile) {
-      is = 0;
-      itile += gridDim.x;
-    }
+    advance(ic);
   };
 
   for (int64_t j = 0; j < S - 1 && j < J; ++j) issue(j);
@@ -228,8 +274,7 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
   float hr[N], hp = 0.f;  // gates of this lane's token for stream n
 #pragma unroll
   for (int jj = 0; jj < N; ++jj) hr[jj] = 0.f;
-  int64_t ctile = blockIdx.x;
-  int cs = 0;  // stage being consumed
+  Cursor cc = start();  // stage being consumed
   for (int64_t j = 0; j < J; ++j) {
     // this wave's loads of stage j have landed (see VM_C); near the end
     // fewer stages follow it and everything is waited for
@@ -245,16 +290,17 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     const uint32_t slot = lds_addr(ring) + (uint32_t)((j % S) * kPPUnits * 1024);
-    const int64_t tb = ctile * TT;
+    const int64_t tb = cc.tile * TT;
     const int nv = (int)(T - tb < TT ? T - tb : TT);
 
-    if (cs < nst_c) {
+    {
       // ---- contraction stage --------------------------------------------
       if (j + S - 1 < J) issue(j + S - 1);
-      if (cs == 0) {
+      if (cc.fresh) {
         // h_res[t][jj][n] (row jj of the token's 64-byte h_res) and h_post[t][n]
         const int tt = 16 * rb + r;
-        const uint32_t ga = gates_lds + (tt >> 4) * 1024 + (tt & 15) * 64 + n * 4;
+        const uint32_t gl = gates_lds + (uint32_t)cc.par * (3 * kWave * 16);
+        const uint32_t ga = gl + (tt >> 4) * 1024 + (tt & 15) * 64 + n * 4;
         asm volatile(
             "ds_read_b32 %0, %5\n\t"
             "ds_read_b32 %1, %5 offset:16\n\t"
@@ -263,7 +309,7 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
             "ds_read_b32 %4, %6\n\t"
             "s_waitcnt lgkmcnt(0)"
             : "=&v"(hr[0]), "=&v"(hr[1]), "=&v"(hr[2]), "=&v"(hr[3]), "=&v"(hp)
-            : "v"(ga), "v"(gates_lds + 2048 + tt * 16 + n * 4)
+            : "v"(ga), "v"(gl + 2048 + tt * 16 + n * 4)
             : "memory");
       }
       // x (streams 0..3) and h_out at columns 64s + 32h + 8c (h = 0, 1) and
@@ -321,7 +367,7 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
 #pragma unroll
         for (int i = 0; i < 4; ++i) S1[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)A[1][i], kDppRor8, 0xF, 0xF, false);
         const auto rxn = rows_rsrc(a.x_next + tb * K, (int64_t)nv * K * 2);
-        const uint32_t d2 = (uint32_t)(cs * kPPCW * 2);
+        const uint32_t d2 = (uint32_t)(cc.s * kPPCW * 2);
         u32x4 W0, W1;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -348,13 +394,13 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[mt] += part[mt];
 
-      if (cs == nst_c - 1) {
-        // ---- tile's mixes (partials added in a fixed order), heads, Sinkhorn
+      if (cc.s == nst - 1 || j == J - 1) {
+        // ---- the run's sums of the tile (partials added in a fixed order) --
         // acc: lane (r, c) holds token 16rb + 4c + v, m = 16mt + r; after the
         // shuffles the lanes of row r hold sum(x_next^2) of token 16rb + r
-        // over this wave's streams and columns.  The slot of this stage is
-        // free once every wave has read it (first barrier) and serves as the
-        // exchange buffer: [rb][part_k - 1][mt][lane].
+        // over this wave's stream.  The slot of this stage is free once every
+        // wave has read it (first barrier) and serves as the exchange buffer
+        // [rb][part_k - 1][mt][lane] until the barrier of the next stage.
         ssq += __shfl_xor(ssq, 16, kWave);
         ssq += __shfl_xor(ssq, 32, kWave);
         __syncthreads();
@@ -366,65 +412,73 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
         }
         __syncthreads();
         if (part_k == 0) {
-          float ssq_t = ssq;
 #pragma unroll
           for (int k = 0; k < 3; ++k) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) acc[mt] += xch[((rb * 3 + k) * MT + mt) * kWave + lane];
-            ssq_t += red_ssq[rb][k][r];
+            ssq += red_ssq[rb][k][r];
           }
-          const float inv_row = 1.0f / sqrtf(ssq_t / (float)K + a.norm_eps);
+          if constexpr (HEADS) {
+            const float inv_row = 1.0f / sqrtf(ssq / (float)K + a.norm_eps);
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float inv = __shfl(inv_row, 4 * q + v, kWave);
-            const int tt = 16 * rb + 4 * q + v;
+            for (int v = 0; v < 4; ++v) {
+              const float inv = __shfl(inv_row, 4 * q + v, kWave);
+              const int tt = 16 * rb + 4 * q + v;
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              if (16 * mt + r < M) mix_sh[tt][16 * mt + r] = acc[mt][v] * inv;
+              for (int mt = 0; mt < MT; ++mt)
+                if (16 * mt + r < M) mix_sh[tt][16 * mt + r] = acc[mt][v] * inv;
+            }
+            if (q == 0) inv_sh[16 * rb + r] = inv_row;
+          } else {
+            const int64_t at = (cc.tile < left0 ? 0 : (int64_t)blockIdx.x - (cc.tile - left0) * nst / a.w) * T + tb + 16 * rb;
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+              for (int mt = 0; mt < MT; ++mt)
+                if (16 * rb + 4 * q + v < nv && 16 * mt + r < M) a.part[(at + 4 * q + v) * M + 16 * mt + r] = acc[mt][v];
+            if (q == 0 && 16 * rb + r < nv) a.part_ssq[at + r] = ssq;
           }
-          if (q == 0) inv_sh[16 * rb + r] = inv_row;
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
         ssq = 0.f;
-        __syncthreads();
-        if (a.mixes) {
-          for (int idx = tid; idx < TT * M; idx += kPPThreads) {
-            const int tt = idx / M, m = idx - (idx / M) * M;
-            if (tt < nv) a.mixes[(tb + tt) * M + m] = mix_sh[tt][m];
-          }
-        }
-        if (a.inv_rms && tid < nv) a.inv_rms[tb + tid] = inv_sh[tid];
-        static_assert(kPPThreads / L == TT, "one pass of heads and Sinkhorn");
-        {
-          const int tt = tid / L;
-          const int64_t tok = tb + tt;
-          const bool ok = tt < nv;
-          const float logit = mix_sh[tt][2 * N + e] * a2 + base_l;
-          const float lc = clamp_logit(logit, a.apply_clamp, a.cmin, a.cmax);
-          const float c = sinkhorn_fwd<N>(lc, a.hc_eps, a.iters);
-          if (ok) {
-            a.comb[tok * L + e] = c;
-            if (a.logits) a.logits[tok * L + e] = logit;
-          }
-          if (e < N) {
-            const float p = sigmoidf_(mix_sh[tt][e] * a0 + base_h) + a.hc_eps;
-            if (ok) {
-              a.pre_ws[tok * N + e] = p;
-              if (a.pre) a.pre[tok * N + e] = p;
+        if constexpr (HEADS) {
+          __syncthreads();
+          if (a.mixes) {
+            for (int idx = tid; idx < TT * M; idx += kPPThreads) {
+              const int tt = idx / M, m = idx - (idx / M) * M;
+              if (tt < nv) a.mixes[(tb + tt) * M + m] = mix_sh[tt][m];
             }
-          } else if (e < 2 * N) {
-            const float po = 2.0f * sigmoidf_(mix_sh[tt][e] * a1 + base_h);
-            if (ok) a.post_out[tok * N + (e - N)] = po;
           }
+          if (a.inv_rms && tid < nv) a.inv_rms[tb + tid] = inv_sh[tid];
+          static_assert(kPPThreads / L == TT, "one pass of heads and Sinkhorn");
+          {
+            const int tt = tid / L;
+            const int64_t tok = tb + tt;
+            const bool ok = tt < nv;
+            const float logit = mix_sh[tt][2 * N + e] * a2 + base_l;
+            const float lc = clamp_logit(logit, a.apply_clamp, a.cmin, a.cmax);
+            const float c = sinkhorn_fwd<N>(lc, a.hc_eps, a.iters);
+            if (ok) {
+              a.comb[tok * L + e] = c;
+              if (a.logits) a.logits[tok * L + e] = logit;
+            }
+            if (e < N) {
+              const float p = sigmoidf_(mix_sh[tt][e] * a0 + base_h) + a.hc_eps;
+              if (ok) {
+                a.pre_ws[tok * N + e] = p;
+                if (a.pre) a.pre[tok * N + e] = p;
+              }
+            } else if (e < 2 * N) {
+              const float po = 2.0f * sigmoidf_(mix_sh[tt][e] * a1 + base_h);
+              if (ok) a.post_out[tok * N + (e - N)] = po;
+            }
+          }
+          __syncthreads();
         }
-        __syncthreads();
       }
     }
-    if (++cs == per_tile) {
-      cs = 0;
-      ctile += gridDim.x;
-    }
+    advance(cc);
   }
 }
 
@@ -441,8 +495,41 @@ bool post_pre_usable(const void* x, const void* h_out, const void* phi, const vo
 
 using namespace mhc;
 
+namespace {
+// One block a CU (its LDS).  Whole tiles in rounds over all CUs, in an order
+// that keeps the blocks on neighbouring tiles (runs of several tiles a block
+// were 10% slower at D = 2048), then runs of equal length over the tiles left;
+// at most about 64 slots of sums a tile for the finish kernel to add.
+struct PostPrePlan {
+  int64_t w = 1, blocks = 0;
+  int rounds = 0;
+  bool whole_rounds = false;
+  size_t ssq_off = 0, y_off = 0, bytes = 0;
+};
+PostPrePlan post_pre_plan(int64_t T, int32_t D) {
+  PostPrePlan p;
+  if (T <= 0) return p;
+  const int64_t nst = D / kPPCW, ntiles = (T + kPPTile - 1) / kPPTile, cus = device_cu_count();
+  p.rounds = (int)(ntiles / cus);
+  const int64_t total = (ntiles - p.rounds * cus) * nst;
+  p.w = (total + cus - 1) / cus;
+  if (p.w < (nst + 63) / 64) p.w = (nst + 63) / 64;
+  p.blocks = p.rounds ? cus : (total + p.w - 1) / p.w;
+  p.whole_rounds = total == 0;
+  int64_t slots = total ? (nst + p.w - 1) / p.w + 1 : 1;
+  if (slots > p.blocks) slots = p.blocks;
+  p.ssq_off = align256((size_t)slots * T * kPPM * 4);
+  p.y_off = p.ssq_off + align256((size_t)slots * T * 4);
+  p.bytes = p.y_off + fwd_y_ws_bytes(T, kPPN);
+  return p;
+}
+}  // namespace
+
 extern "C" size_t mhc_post_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, int32_t phi_dtype) {
-  return mhc_pre_fwd_workspace_size(T, N, D, phi_dtype);
+  const size_t pre = mhc_pre_fwd_workspace_size(T, N, D, phi_dtype);
+  if (N != kPPN || phi_dtype != MHC_DTYPE_BF16 || D < kPPMinD || D % kPPCW || T <= 0) return pre;
+  const size_t own = post_pre_plan(T, D).bytes;
+  return own > pre ? own : pre;
 }
 
 extern "C" int mhc_post_pre_fwd_ex(const void* x, const float* h_res, const void* h_out, const float* h_post,
@@ -470,8 +557,9 @@ extern "C" int mhc_post_pre_fwd_ex(const void* x, const float* h_res, const void
                                             (hipStream_t)stream, &used);
     if (rc || used) return rc;
   }
-  if (!post_pre_usable(x, h_out, phi, x_next, y, x_dtype, phi_dtype, N, D) || !workspace ||
-      workspace_bytes < fwd_y_ws_bytes(T, N) ||
+  const bool usable = post_pre_usable(x, h_out, phi, x_next, y, x_dtype, phi_dtype, N, D);
+  const PostPrePlan p = usable ? post_pre_plan(T, D) : PostPrePlan{};
+  if (!usable || !workspace || workspace_bytes < p.bytes ||
       pre_fwd_single_pass_applies(x_next, x_dtype, phi, phi_dtype, y, workspace_bytes, T, N, D,
                                   (hipStream_t)stream)) {
     // every other shape, and where the pre forward reads x_next once (its
@@ -490,31 +578,65 @@ extern "C" int mhc_post_pre_fwd_ex(const void* x, const float* h_res, const void
   a.h_out = static_cast<const bf16_t*>(h_out);
   a.h_post = h_post;
   a.phi = static_cast<const uint16_t*>(phi);
-  a.alpha = alpha;
-  a.base = base;
-  a.norm_eps = norm_eps;
-  a.hc_eps = hc_eps;
-  a.cmin = clamp_min;
-  a.cmax = clamp_max;
-  a.apply_clamp = (clamp_min != 0.0f || clamp_max != 0.0f) ? 1 : 0;
-  a.iters = iter_times;
   a.x_next = static_cast<bf16_t*>(x_next);
-  a.y = static_cast<bf16_t*>(y);
-  a.post_out = post_out;
-  a.comb = comb_frag;
-  a.inv_rms = inv_rms;
-  a.mixes = mixes;
-  a.logits = h_res_logits;
-  a.pre = pre;
-  a.pre_ws = static_cast<float*>(workspace);
+  char* ws = static_cast<char*>(workspace);
+  a.part = reinterpret_cast<float*>(ws);
+  a.part_ssq = reinterpret_cast<float*>(ws + p.ssq_off);
+  a.w = p.w;
+  a.rounds = p.rounds;
   a.T = T;
   a.D = D;
-  const int64_t ntiles = (T + kPPTile - 1) / kPPTile;
-  const int64_t cus = device_cu_count();
-  const int64_t grid = ntiles < cus ? ntiles : cus;  // one block per CU (LDS ring)
-  hipLaunchKernelGGL(post_pre_fwd_kernel, dim3((unsigned)grid), dim3(kPPThreads), 0, (hipStream_t)stream, a);
+  const bool heads = p.whole_rounds;
+  if (heads) {
+    a.alpha = alpha;
+    a.base = base;
+    a.norm_eps = norm_eps;
+    a.hc_eps = hc_eps;
+    a.cmin = clamp_min;
+    a.cmax = clamp_max;
+    a.apply_clamp = (clamp_min != 0.0f || clamp_max != 0.0f) ? 1 : 0;
+    a.iters = iter_times;
+    a.post_out = post_out;
+    a.comb = comb_frag;
+    a.inv_rms = inv_rms;
+    a.mixes = mixes;
+    a.logits = h_res_logits;
+    a.pre = pre;
+    a.pre_ws = reinterpret_cast<float*>(ws);
+    hipLaunchKernelGGL(post_pre_fwd_kernel<true>, dim3((unsigned)p.blocks), dim3(kPPThreads), 0, (hipStream_t)stream,
+                       a);
+    if (int rc = check_launch("post_pre_fwd")) return rc;
+    return launch_pre_y_pass(x_next, a.pre_ws, y, T, N, D, (hipStream_t)stream);
+  }
+  hipLaunchKernelGGL(post_pre_fwd_kernel<false>, dim3((unsigned)p.blocks), dim3(kPPThreads), 0, (hipStream_t)stream,
+                     a);
   if (int rc = check_launch("post_pre_fwd")) return rc;
-  return launch_pre_y_pass(x_next, a.pre_ws, y, T, N, D, (hipStream_t)stream);
+  PreFinish f{};
+  f.x = x_next;
+  f.part = a.part;
+  f.part_ssq = a.part_ssq;
+  f.ws = ws + p.y_off;
+  f.nst = D / kPPCW;
+  f.tt = kPPTile;
+  f.w = p.w;
+  f.whole = p.rounds * p.blocks;
+  f.alpha = alpha;
+  f.base = base;
+  f.norm_eps = norm_eps;
+  f.hc_eps = hc_eps;
+  f.cmin = clamp_min;
+  f.cmax = clamp_max;
+  f.iters = iter_times;
+  f.y = y;
+  f.post_out = post_out;
+  f.comb = comb_frag;
+  f.inv_rms = inv_rms;
+  f.mixes = mixes;
+  f.logits = h_res_logits;
+  f.pre = pre;
+  f.T = T;
+  f.D = D;
+  return launch_pre_finish(f, (hipStream_t)stream);
 }
 
 extern "C" int mhc_post_pre_fwd(const void* x, const float* h_res, const void* h_out, const float* h_post,

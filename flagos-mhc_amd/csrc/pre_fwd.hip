@@ -70,6 +70,7 @@ struct PreFwdArgs {
   const void* phi_raw;
   int gen_nst, gen_tt;
   int64_t gen_w;
+  int64_t gen_whole;  // tiles before the runs, summed by one block each
   // single-pass form: its status word (nonzero when a bounded wait timed
   // out); the finalize kernel then writes NaN to every output of the call
   // and copies the word to status_out (the caller's, may be null)
@@ -868,7 +869,8 @@ __global__ __launch_bounds__(kKsThreads) void pre_fwd_ks8_kernel(PreFwdArgs a) {
 // contraction, the blocks whose runs touch the token's tile.
 __device__ __forceinline__ int fwd_slots(const PreFwdArgs& a, int64_t tok, int nsplit) {
   if (!a.gen_w) return nsplit;
-  const int64_t tile = tok / a.gen_tt;
+  const int64_t tile = tok / a.gen_tt - a.gen_whole;
+  if (tile < 0) return 1;
   return (int)(((tile + 1) * a.gen_nst - 1) / a.gen_w - tile * a.gen_nst / a.gen_w) + 1;
 }
 
@@ -1206,6 +1208,42 @@ static int dispatch_pre_fwd(int N, const PreFwdArgs& a, bool vec, hipStream_t st
     case 8: return launch_pre_fwd<8, S>(a, vec, st);
   }
   return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_fwd: N=%d not supported (4, 8)", N);
+}
+
+int launch_pre_finish(const PreFinish& f, hipStream_t st) {
+  PreFwdArgs a{};
+  a.x = f.x;
+  a.part = f.part;
+  a.part_ssq = f.part_ssq;
+  a.pre_ws = reinterpret_cast<float*>(f.ws);
+  a.inv_ws = reinterpret_cast<float*>(f.ws + align256((size_t)f.T * 4 * 4));
+  a.gen_nst = f.nst;
+  a.gen_tt = f.tt;
+  a.gen_w = f.w;
+  a.gen_whole = f.whole;
+  a.alpha = f.alpha;
+  a.base = f.base;
+  a.norm_eps = f.norm_eps;
+  a.hc_eps = f.hc_eps;
+  a.cmin = f.cmin;
+  a.cmax = f.cmax;
+  a.apply_clamp = (f.cmin != 0.0f || f.cmax != 0.0f) ? 1 : 0;
+  a.iters = f.iters;
+  a.y = f.y;
+  a.post_out = f.post_out;
+  a.comb = f.comb;
+  a.inv_rms = f.inv_rms;
+  a.mixes = f.mixes;
+  a.logits = f.logits;
+  a.pre = f.pre;
+  a.T = f.T;
+  a.D = f.D;
+  if (finish_applies(a.T, 4, a.D)) return launch_pre_fwd_finish<4, bf16_t>(a, 0, st);
+  constexpr int TPP = kFwdThreads / 16;
+  hipLaunchKernelGGL((pre_fwd_finalize_kernel<4>), dim3((unsigned)((a.T + TPP - 1) / TPP)), dim3(kFwdThreads), 0, st,
+                     a, 0);
+  if (int rc = check_launch("pre_fwd_finalize")) return rc;
+  return launch_pre_fwd_y<4>(a, st);
 }
 
 template <int N>

@@ -397,15 +397,15 @@ __device__ __forceinline__ void gen_y8(const PreFwdArgs& a, int64_t t, int c0, i
 }
 
 // One block per token, after the general contraction or the LDS-pipelined
-// kernels' sums (see finish_applies).  All waves add the
-// slots, wave 0 then runs the heads and Sinkhorn while the others form y from
-// rows they began to load before the sums were complete; y needs only the
-// pre gates, which every wave forms for itself.
+// kernels' sums (see finish_applies).  All waves add the slots, wave 0 then
+// runs the heads and Sinkhorn while the others form y from rows they began to
+// load before the sums were complete; y needs only the pre gates, which every
+// wave forms for itself, a gate a lane.
 constexpr int kFinishWaves = 16;
 template <int N, typename S, bool XS>
 __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_finish_kernel(PreFwdArgs a, int nsplit) {
   constexpr int M = PreDims<N>::M, L = N * N, VP = N == 4 ? 32 : 128;  // VP > M: the sums and the sum of squares
-  static_assert(M < VP, "a lane for each sum");
+  static_assert(M < VP && VP <= 2 * kWave, "a lane for each sum; blocks of at least two waves");
   __shared__ float red[kWave * kFinishWaves / VP][VP];
   __shared__ float tot[VP];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -422,7 +422,7 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_finish_kernel(Pr
 #pragma unroll 4
       for (int s = g; s < ns; s += groups) sum += p[s * stride];
     }
-    red[g][v] = sum;
+    if (g < groups) red[g][v] = sum;
   }
   const int first = (wave - 1) * 512;
   Raw8<S> X[N];
@@ -434,12 +434,12 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_finish_kernel(Pr
     tot[tid] = sum;
   }
   __syncthreads();
-  const float inv = rms_inv(tot[M], (float)(N * (int64_t)a.D), a.norm_eps);
-  const float a0 = a.alpha[0];
+  const float inv = rms_inv(tot[M], (float)(N * (int64_t)a.D), a.norm_eps), a0 = a.alpha[0];
   if (wave > 0) {
+    const float p_l = pre_gate(tot[lane % N] * inv, a0, a.base[lane % N], a.hc_eps);
     float p[N];
 #pragma unroll
-    for (int n = 0; n < N; ++n) p[n] = pre_gate(tot[n] * inv, a0, a.base[n], a.hc_eps);
+    for (int n = 0; n < N; ++n) p[n] = __shfl(p_l, n, kWave);
     for (int c0 = first; c0 < a.D; c0 += yw * 512) {
       if (c0 != first) gen_load_rows<N, S, XS>(a, t, c0, lane, X);
       gen_y8<N, S, XS>(a, t, c0, lane, X, p, inv);
@@ -488,15 +488,17 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_gen_y_kernel(Pre
 
 // ---- host side --------------------------------------------------------------
 // Whether the finish kernel ends a call, rather than the finalize kernel
-// (tokens packed N * N lanes each) and a y kernel.  Its Sinkhorn wave per token
-// hides behind the token's y only where that is long enough, or where so few
-// tokens run that a launch less is what counts.  Measured (bf16, us, finish /
-// finalize + y, whole operator): N = 4: D = 256 T = 2048 14.2 / 13.0, T =
-// 16384 39.9 / 25.8; D = 512 T = 4096 16.5 / 17.6, T = 16384 41.9 / 37.9; D =
-// 1024 T = 16384 66.6 / 67.4; D = 5120 257 / 265; T = 64 D = 7168 11.6 / 16.1.
-// N = 8: D = 256 T = 16384 78.2 / 59.5; D = 512 78.3 / 86.3; D = 2048 T =
-// 32768 417 / 430.
-static bool finish_applies(int64_t T, int N, int D) { return T <= 1024 || D >= (N == 8 ? 512 : T <= 4096 ? 512 : 1024); }
+// (tokens packed N * N lanes each) and a y kernel.  Its Sinkhorn chain, about
+// 5 us a token, hides behind other blocks only while there are few of them or
+// each has much y to form; a launch less is what counts at few tokens.
+// Measured (bf16, us, finish / finalize + y, whole operator): N = 4: T = 64 D =
+// 7168 11.6 / 16.2; T = 512 D = 4096 15.0 / 18.0; T = 2048 D = 4096 37.0 / 37.6,
+// D = 256 13.5 / 12.9; T = 16384 D = 256 39 / 26, D = 512 41 / 38, D = 9216 451
+// / 438; fp16 T = 8192 D = 1003 59.6 / 50.5.  N = 8: T = 64 D = 2048 13.6 /
+// 16.1; T = 16384 D = 2048 253 / 262, D = 256 72 / 57.  Four tokens a block
+// (N = 4, one Sinkhorn wave for the four) gained 0 to 6% above 2048 tokens and
+// lost as much at wide rows.
+static bool finish_applies(int64_t T, int N, int D) { return T <= 1024 || (D >= 512 && (N == 8 || T <= 2048)); }
 
 constexpr int kGenSmallT = 64;   // tokens up to which the 16-token tiles run
 constexpr int kGenFewUnits = 128;  // .. and stages of 128-token tiles below which they do

@@ -36,6 +36,27 @@ inline size_t phiT_planes_bytes(int32_t phi_dtype, int M, int64_t K) {
 // x_next.
 int launch_pre_y_pass(const void* x, const float* pre, void* y, int64_t T, int N, int D, hipStream_t st);
 
+// The pre forward's last step for N = 4, bf16 x (T, N, D) with D % 8 == 0 and
+// 16-byte aligned rows: a token's sums in slots (runs of `w` stages, `nst`
+// stages a tile of `tt` tokens: the blocks whose runs touch the token's tile),
+// then heads, Sinkhorn and y.  `ws`: fwd_y_ws_bytes of scratch.  The fused
+// post + pre forward runs it on x_next.  The first `whole` tiles have one slot.
+struct PreFinish {
+  const void* x;
+  float *part, *part_ssq;  // [slot][T][24], [slot][T]
+  char* ws;
+  int nst, tt;
+  int64_t w, whole;
+  const float *alpha, *base;
+  float norm_eps, hc_eps, cmin, cmax;
+  int iters;
+  void* y;
+  float *post_out, *comb, *inv_rms, *mixes, *logits, *pre;
+  int64_t T;
+  int D;
+};
+int launch_pre_finish(const PreFinish& f, hipStream_t st);
+
 // Whether mhc_pre_fwd without x_scaled runs its single-pass form (x read
 // from HBM once) on these arguments: N = 4, bf16 x and phi, a slice
 // geometry for D, T large enough, workspace for it, no stream capture.
