@@ -143,6 +143,44 @@ __device__ __forceinline__ void st16nt(void* p, const u32x4& v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
+// The same at any alignment (unaligned 16-byte accesses are single
+// instructions on this part) ..
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 ld16nt_u(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2*>(p));
+}
+__device__ __forceinline__ void st16nt_u(void* p, const u32x4& v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a2*>(p));
+}
+// .. and element by element for a whole row of D < VEC elements (those past it
+// read zero and are not written).
+template <typename S>
+__device__ __forceinline__ u32x4 ld16_elems(const S* row, int D) {
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if constexpr (sizeof(S) == 2) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < D) v[i / 2] |= (uint32_t)reinterpret_cast<const uint16_t*>(row)[i] << (16 * (i & 1));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < D) v[i] = reinterpret_cast<const uint32_t*>(row)[i];
+  }
+  return v;
+}
+template <typename S>
+__device__ __forceinline__ void st16_elems(S* row, int D, const u32x4& v) {
+  if constexpr (sizeof(S) == 2) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < D) reinterpret_cast<uint16_t*>(row)[i] = (uint16_t)(v[i / 2] >> (16 * (i & 1)));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < D) reinterpret_cast<uint32_t*>(row)[i] = v[i];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // XCD-contiguous work order.  Workgroups are dispatched round robin over the
 // eight XCDs (workgroup b runs on XCD b % 8); xcd_contig maps b to an item so

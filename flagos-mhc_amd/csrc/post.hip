@@ -16,7 +16,9 @@
 // scalar loads, every lane streams 16-byte vectors of each of the N rows
 // (non-temporal loads: each input is read once), accumulates in fp32 and
 // stores with round-to-nearest-even (streaming stores: outputs are not
-// re-read here).  The backward's N*N + N dot products
+// re-read here).  Rows at other alignments take unaligned 16-byte accesses
+// (before, element by element: fp16, N = 4, D = 1003, T = 8192 55 -> 31 us
+// forward, 51 -> 44 backward; bf16 D = 907, T = 16384 106 -> 55, 102 -> 77).  The backward's N*N + N dot products
 // are reduced across the wave (and the block) once per token and written by
 // plain stores (no atomics), so results are deterministic.
 #include <type_traits>
@@ -58,6 +60,25 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
 
   const int64_t xrow = t * (int64_t)N * D;
   const int64_t hrow = t * (int64_t)D;
+  // VECTOR: rows of whole 16-byte pieces, 16-byte aligned.  Otherwise the last
+  // lane of a row takes its last V elements again instead of a piece that ends
+  // outside it: it stores the same values twice, and the dot products leave
+  // the `dup` elements out that the lane before it has (rows of less than V
+  // elements go one by one).
+  auto ld = [D](const S* row, int d) {
+    if constexpr (VECTOR)
+      return ld16nt(row + d);
+    else
+      return D < Store<S>::VEC ? ld16_elems(row, D) : ld16nt_u(row + d);
+  };
+  auto st = [D](S* row, int d, const u32x4& v) {
+    if constexpr (VECTOR)
+      st16nt(row + d, v);
+    else if (D < Store<S>::VEC)
+      st16_elems(row, D, v);
+    else
+      st16nt_u(row + d, v);
+  };
 
   if constexpr (VECTOR && N == 8 && std::is_same<S, bf16_t>::value && !SUM) {
     // N = 8: the N*N + N dot products take v_dot2_f32_bf16 on the packed
@@ -109,24 +130,25 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
         for (int i = 0; i < N; ++i) acc_p[i] = dot2(hraw[w], graw[i][w], acc_p[i]);
       }
     }
-  } else if constexpr (VECTOR) {
+  } else {
     constexpr int V = Store<S>::VEC;
-    for (int d = lane * V; d < D; d += kWave * V) {
+    for (int d0 = lane * V; d0 < D; d0 += kWave * V) {
+      const int d = VECTOR || d0 + V <= D || D < V ? d0 : D - V, dup = d0 - d;
       float gv[N][V], xv[N][V], hv[V];
 #pragma unroll
-      for (int i = 0; i < N; ++i) Store<S>::unpack(ld16nt(gy + xrow + (int64_t)i * D + d), gv[i]);
+      for (int i = 0; i < N; ++i) Store<S>::unpack(ld(gy + xrow + (int64_t)i * D, d), gv[i]);
       if constexpr (SUM) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
           float g2[V];
-          Store<S>::unpack(ld16nt(gy2 + xrow + (int64_t)i * D + d), g2);
+          Store<S>::unpack(ld(gy2 + xrow + (int64_t)i * D, d), g2);
 #pragma unroll
           for (int e = 0; e < V; ++e) gv[i][e] += g2[e];
         }
       }
 #pragma unroll
-      for (int j = 0; j < N; ++j) Store<S>::unpack(ld16nt(x + xrow + (int64_t)j * D + d), xv[j]);
-      Store<S>::unpack(ld16nt(h_out + hrow + d), hv);
+      for (int j = 0; j < N; ++j) Store<S>::unpack(ld(x + xrow + (int64_t)j * D, d), xv[j]);
+      Store<S>::unpack(ld(h_out + hrow, d), hv);
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         float o[V];
@@ -137,7 +159,7 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
           for (int i = 0; i < N; ++i) a = fmaf(hr[j * N + i], gv[i][e], a);
           o[e] = a;
         }
-        st16nt(gx + xrow + (int64_t)j * D + d, Store<S>::pack(o));
+        st(gx + xrow + (int64_t)j * D, d, Store<S>::pack(o));
       }
       float oh[V];
 #pragma unroll
@@ -147,7 +169,18 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
         for (int i = 0; i < N; ++i) a = fmaf(hp[i], gv[i][e], a);
         oh[e] = a;
       }
-      st16nt(g_hout + hrow + d, Store<S>::pack(oh));
+      st(g_hout + hrow, d, Store<S>::pack(oh));
+      if constexpr (!VECTOR) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          if (e >= dup) continue;
+#pragma unroll
+          for (int i = 0; i < N; ++i) gv[i][e] = 0.f;
+#pragma unroll
+          for (int j = 0; j < N; ++j) xv[j][e] = 0.f;
+          hv[e] = 0.f;
+        }
+      }
 #pragma unroll
       for (int e = 0; e < V; ++e) {
 #pragma unroll
@@ -157,35 +190,6 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
 #pragma unroll
         for (int i = 0; i < N; ++i) acc_p[i] = fmaf(hv[e], gv[i][e], acc_p[i]);
       }
-    }
-  } else {
-    for (int d = lane; d < D; d += kWave) {
-      float gv[N], xv[N];
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        gv[i] = load_elem(gy, xrow + (int64_t)i * D + d);
-        if constexpr (SUM) gv[i] += load_elem(gy2, xrow + (int64_t)i * D + d);
-      }
-#pragma unroll
-      for (int j = 0; j < N; ++j) xv[j] = load_elem(x, xrow + (int64_t)j * D + d);
-      const float hv = load_elem(h_out, hrow + d);
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        float a = 0.f;
-#pragma unroll
-        for (int i = 0; i < N; ++i) a = fmaf(hr[j * N + i], gv[i], a);
-        store_elem(gx, xrow + (int64_t)j * D + d, a);
-      }
-      float a = 0.f;
-#pragma unroll
-      for (int i = 0; i < N; ++i) a = fmaf(hp[i], gv[i], a);
-      store_elem(g_hout, hrow + d, a);
-#pragma unroll
-      for (int j = 0; j < N; ++j)
-#pragma unroll
-        for (int i = 0; i < N; ++i) acc_r[j * N + i] = fmaf(xv[j], gv[i], acc_r[j * N + i]);
-#pragma unroll
-      for (int i = 0; i < N; ++i) acc_p[i] = fmaf(hv, gv[i], acc_p[i]);
     }
   }
 
@@ -229,11 +233,17 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
 constexpr int kPostBlockWaves = 8;     // backward: 132 VGPRs at N = 4 allow 8 waves
 constexpr int kPostFwdBlockWaves = 16;  // forward: 68 VGPRs
 
+template <typename S>
+__host__ __device__ constexpr int post_fwd_vec(bool vec) {
+  return vec || sizeof(S) == 2 ? Store<S>::VEC : 1;
+}
 template <int N, typename S, bool VECTOR>
 __global__ __launch_bounds__(kWave * kPostFwdBlockWaves) void post_fwd_block_kernel(
     const S* __restrict__ x, const float* __restrict__ h_res, const S* __restrict__ h_out,
     const float* __restrict__ h_post, S* __restrict__ y, int D) {
-  constexpr int V = VECTOR ? Store<S>::VEC : 1, CW = kWave * V;
+  // unaligned fp32 rows: element loads, which coalesce as they are (N = 8, D =
+  // 515: 47 us against 57 for unaligned 16-byte pieces at T = 8192; N = 4 equal)
+  constexpr int V = post_fwd_vec<S>(VECTOR), CW = kWave * V;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int W = blockDim.x / kWave;
@@ -246,12 +256,32 @@ __global__ __launch_bounds__(kWave * kPostFwdBlockWaves) void post_fwd_block_ker
 #pragma unroll
   for (int i = 0; i < N; ++i) hp[i] = h_post[t * N + i];
   const int64_t xrow = t * (int64_t)N * D, hrow = t * (int64_t)D;
-  for (int d = wave * CW + lane * V; d < D; d += W * CW) {
+  // VECTOR: rows of whole 16-byte pieces, 16-byte aligned.  Otherwise the last
+  // lane of a row takes its last V elements again instead of a piece that ends
+  // outside it: it stores the same values twice, and the dot products leave
+  // the `dup` elements out that the lane before it has (rows of less than V
+  // elements go one by one).
+  auto ld = [D](const S* row, int d) {
+    if constexpr (VECTOR)
+      return ld16nt(row + d);
+    else
+      return D < Store<S>::VEC ? ld16_elems(row, D) : ld16nt_u(row + d);
+  };
+  auto st = [D](S* row, int d, const u32x4& v) {
+    if constexpr (VECTOR)
+      st16nt(row + d, v);
+    else if (D < Store<S>::VEC)
+      st16_elems(row, D, v);
+    else
+      st16nt_u(row + d, v);
+  };
+  for (int d0 = wave * CW + lane * V; d0 < D; d0 += W * CW) {
+    const int d = VECTOR || d0 + V <= D || D < V ? d0 : D - V;
     float xv[N][V], hv[V];
-    if constexpr (VECTOR) {
+    if constexpr (V > 1) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) Store<S>::unpack(ld16nt(x + xrow + (int64_t)j * D + d), xv[j]);
-      Store<S>::unpack(ld16nt(h_out + hrow + d), hv);
+      for (int j = 0; j < N; ++j) Store<S>::unpack(ld(x + xrow + (int64_t)j * D, d), xv[j]);
+      Store<S>::unpack(ld(h_out + hrow, d), hv);
     } else {
 #pragma unroll
       for (int j = 0; j < N; ++j) xv[j][0] = load_elem(x, xrow + (int64_t)j * D + d);
@@ -267,8 +297,8 @@ __global__ __launch_bounds__(kWave * kPostFwdBlockWaves) void post_fwd_block_ker
         for (int j = 0; j < N; ++j) acc = fmaf(hr[j * N + i], xv[j][e], acc);
         o[e] = acc;
       }
-      if constexpr (VECTOR)
-        st16nt(y + xrow + (int64_t)i * D + d, Store<S>::pack(o));
+      if constexpr (V > 1)
+        st(y + xrow + (int64_t)i * D, d, Store<S>::pack(o));
       else
         store_elem(y, xrow + (int64_t)i * D + d, o[0]);
     }
@@ -282,7 +312,7 @@ __global__ __launch_bounds__(kWave * kPostBlockWaves, MINW) void post_bwd_block_
     const S* __restrict__ h_out, const float* __restrict__ h_post, S* __restrict__ gx,
     float* __restrict__ g_hres, S* __restrict__ g_hout, float* __restrict__ g_hpost, int D,
     const S* __restrict__ gy2) {
-  constexpr int V = VECTOR ? Store<S>::VEC : 1, CW = kWave * V, R = N * N + N;
+  constexpr int V = Store<S>::VEC, CW = kWave * V, R = N * N + N;
   __shared__ float red[kPostBlockWaves][R];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -299,33 +329,42 @@ __global__ __launch_bounds__(kWave * kPostBlockWaves, MINW) void post_bwd_block_
 #pragma unroll
   for (int i = 0; i < N; ++i) acc_p[i] = 0.f;
   const int64_t xrow = t * (int64_t)N * D, hrow = t * (int64_t)D;
-  for (int d = wave * CW + lane * V; d < D; d += W * CW) {
+  // VECTOR: rows of whole 16-byte pieces, 16-byte aligned.  Otherwise the last
+  // lane of a row takes its last V elements again instead of a piece that ends
+  // outside it: it stores the same values twice, and the dot products leave
+  // the `dup` elements out that the lane before it has (rows of less than V
+  // elements go one by one).
+  auto ld = [D](const S* row, int d) {
+    if constexpr (VECTOR)
+      return ld16nt(row + d);
+    else
+      return D < Store<S>::VEC ? ld16_elems(row, D) : ld16nt_u(row + d);
+  };
+  auto st = [D](S* row, int d, const u32x4& v) {
+    if constexpr (VECTOR)
+      st16nt(row + d, v);
+    else if (D < Store<S>::VEC)
+      st16_elems(row, D, v);
+    else
+      st16nt_u(row + d, v);
+  };
+  for (int d0 = wave * CW + lane * V; d0 < D; d0 += W * CW) {
+    const int d = VECTOR || d0 + V <= D || D < V ? d0 : D - V, dup = d0 - d;
     float gv[N][V], xv[N][V], hv[V];
-    if constexpr (VECTOR) {
 #pragma unroll
-      for (int i = 0; i < N; ++i) Store<S>::unpack(ld16nt(gy + xrow + (int64_t)i * D + d), gv[i]);
-      if constexpr (SUM) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          float g2[V];
-          Store<S>::unpack(ld16nt(gy2 + xrow + (int64_t)i * D + d), g2);
-#pragma unroll
-          for (int e = 0; e < V; ++e) gv[i][e] += g2[e];
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < N; ++j) Store<S>::unpack(ld16nt(x + xrow + (int64_t)j * D + d), xv[j]);
-      Store<S>::unpack(ld16nt(h_out + hrow + d), hv);
-    } else {
+    for (int i = 0; i < N; ++i) Store<S>::unpack(ld(gy + xrow + (int64_t)i * D, d), gv[i]);
+    if constexpr (SUM) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
-        gv[i][0] = load_elem(gy, xrow + (int64_t)i * D + d);
-        if constexpr (SUM) gv[i][0] += load_elem(gy2, xrow + (int64_t)i * D + d);
-      }
+        float g2[V];
+        Store<S>::unpack(ld(gy2 + xrow + (int64_t)i * D, d), g2);
 #pragma unroll
-      for (int j = 0; j < N; ++j) xv[j][0] = load_elem(x, xrow + (int64_t)j * D + d);
-      hv[0] = load_elem(h_out, hrow + d);
+        for (int e = 0; e < V; ++e) gv[i][e] += g2[e];
+      }
     }
+#pragma unroll
+    for (int j = 0; j < N; ++j) Store<S>::unpack(ld(x + xrow + (int64_t)j * D, d), xv[j]);
+    Store<S>::unpack(ld(h_out + hrow, d), hv);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       float o[V];
@@ -336,10 +375,7 @@ __global__ __launch_bounds__(kWave * kPostBlockWaves, MINW) void post_bwd_block_
         for (int i = 0; i < N; ++i) a = fmaf(hr[j * N + i], gv[i][e], a);
         o[e] = a;
       }
-      if constexpr (VECTOR)
-        st16nt(gx + xrow + (int64_t)j * D + d, Store<S>::pack(o));
-      else
-        store_elem(gx, xrow + (int64_t)j * D + d, o[0]);
+      st(gx + xrow + (int64_t)j * D, d, Store<S>::pack(o));
     }
     float oh[V];
 #pragma unroll
@@ -349,10 +385,18 @@ __global__ __launch_bounds__(kWave * kPostBlockWaves, MINW) void post_bwd_block_
       for (int i = 0; i < N; ++i) a = fmaf(hp[i], gv[i][e], a);
       oh[e] = a;
     }
-    if constexpr (VECTOR)
-      st16nt(g_hout + hrow + d, Store<S>::pack(oh));
-    else
-      store_elem(g_hout, hrow + d, oh[0]);
+    st(g_hout + hrow, d, Store<S>::pack(oh));
+    if constexpr (!VECTOR) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        if (e >= dup) continue;
+#pragma unroll
+        for (int i = 0; i < N; ++i) gv[i][e] = 0.f;
+#pragma unroll
+        for (int j = 0; j < N; ++j) xv[j][e] = 0.f;
+        hv[e] = 0.f;
+      }
+    }
 #pragma unroll
     for (int e = 0; e < V; ++e) {
 #pragma unroll
@@ -694,7 +738,7 @@ static int launch_post_fwd(const void* x, const float* h_res, const void* h_out,
       return check_launch("post_fwd_dma");
     }
   }
-  const int waves = post_block_waves(D, vec ? Store<S>::VEC : 1, kPostFwdBlockWaves);
+  const int waves = post_block_waves(D, post_fwd_vec<S>(vec), kPostFwdBlockWaves);
   const dim3 gs((unsigned)T), bs(kWave * waves);
   // Blocks of 10 or more waves run one token per CU at a time (D = 7168 /
   // 5120: 2.6% / 1.6% faster); narrower ones (N = 8 takes this kernel at
@@ -733,7 +777,7 @@ static int launch_post_bwd(const void* gy, const void* gy2, const void* x, const
   const bool block_form = T < kPostStreamMinT || (N <= 4 && !dma) || (sum && dma);
   const S* g2 = static_cast<const S*>(gy2);
   if (block_form) {
-    const dim3 gs((unsigned)T), bs(kWave * post_block_waves(D, vec ? Store<S>::VEC : 1, kPostBlockWaves));
+    const dim3 gs((unsigned)T), bs(kWave * post_block_waves(D, Store<S>::VEC, kPostBlockWaves));
     if (int rc = check_grid(gs, bs, "mhc_post_bwd")) return rc;
     if (sum) {
       if (vec)

@@ -179,7 +179,6 @@ template <typename S> struct Raw8 { u32x4 v[sizeof(S) / 2]; };
 
 // Global loads and stores of rows at any element alignment: unaligned 16- and
 // 8-byte accesses are single instructions on this part.
-typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 __device__ __forceinline__ u32x4 ld16u(const void* p) { return *reinterpret_cast<const u32x4_a2*>(p); }
 
