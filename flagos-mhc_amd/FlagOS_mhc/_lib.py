@@ -8,7 +8,10 @@ are not on a HIP device, the operators raise instead of computing on the CPU.
 from __future__ import annotations
 
 import collections
+import contextlib
 import ctypes
+import functools
+import math
 import os
 import threading
 
@@ -107,7 +110,39 @@ def ptr(t):
 
 
 def stream_of(t: torch.Tensor):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current HIP stream of t's device."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+_no_guard = contextlib.nullcontext()
+
+
+def on_device(dev: torch.device):
+    """A context in which `dev` is the current device (none is entered where it
+    is already: switching costs a call more than a few microseconds)."""
+    return _no_guard if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
+def operand(t: torch.Tensor, shape, dtype: torch.dtype) -> torch.Tensor:
+    """t as a contiguous tensor of `dtype` with shape's elements in order (the
+    kernels take its address only, so a tensor that already holds them is
+    returned as it is, whatever its own shape)."""
+    if t.dtype == dtype and t.is_contiguous() and t.numel() == math.prod(shape):
+        return t
+    return t.reshape(shape).to(dtype).contiguous()
+
+
+@functools.lru_cache(maxsize=1024)
+def workspace_size(name: str, dev_index: int, *args) -> int:
+    """A *_workspace_size query: a function of the sizes and the device alone."""
+    with torch.cuda.device(dev_index):
+        return int(getattr(load(), name)(*args))
+
+
+def workspace(name: str, dev: torch.device, *args):
+    """(tensor, bytes) of scratch for a call on `dev`."""
+    n = workspace_size(name, dev.index, *args)
+    return torch.empty((max(n, 1),), dtype=torch.uint8, device=dev), n
 
 
 def require_device(what: str, *tensors) -> None:
@@ -172,6 +207,8 @@ class SinglePassStatus:
             self._pending.append((slot, ev))
 
     def check(self, block: bool) -> None:
+        if not self._pending:  # nothing reported since the last check
+            return
         if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
             return
         with self._lock:

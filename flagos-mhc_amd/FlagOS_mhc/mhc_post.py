@@ -34,26 +34,36 @@ def _flatten_bsn(x, h_res, h_out, h_post):
     raise ValueError(f"unsupported x.dim()={x.dim()}, expect 3 or 4")
 
 
+def _tokens(x):
+    """(T, N, D) of a (B, S, N, D) or (T, N, D) tensor."""
+    if x.dim() == 4:
+        B, S, N, D = x.shape
+        return B * S, N, D
+    if x.dim() == 3:
+        return tuple(x.shape)
+    raise ValueError(f"unsupported x.dim()={x.dim()}, expect 3 or 4")
+
+
 def mhc_post(x, h_res, h_out, h_post):
     """Forward of mhc_post on the HIP device (no CPU fallback)."""
     _lib.require_device("mhc_post", x, h_res, h_out, h_post)
-    xf, hres, hout, hpost, shape = _flatten_bsn(x, h_res, h_out, h_post)
-    T, N, D = xf.shape
+    T, N, D = _tokens(x)
+    xf = x.contiguous()
+    hres = _lib.operand(h_res, (T, N, N), torch.float32)
+    hout = _lib.operand(h_out, (T, D), xf.dtype)
+    hpost = _lib.operand(h_post, (T, N), torch.float32)
     if N not in SUPPORTED_N:
         raise NotImplementedError(f"mhc_post: N={N} not supported (supported: {SUPPORTED_N})")
     code = _lib.dtype_code("mhc_post", xf.dtype)
-    hres = hres.to(torch.float32).contiguous()
-    hpost = hpost.to(torch.float32).contiguous()
-    hout = hout.to(xf.dtype).contiguous()
-    out = torch.empty_like(xf)
+    out = torch.empty_like(xf, memory_format=torch.contiguous_format)
     if T > 0:
         lib = _lib.load()
-        with torch.cuda.device(xf.device):
+        with _lib.on_device(xf.device):
             rc = lib.mhc_post_fwd(xf.data_ptr(), hres.data_ptr(), hout.data_ptr(),
                                   hpost.data_ptr(), out.data_ptr(), T, N, D, code,
                                   _lib.stream_of(xf))
         _lib.check(rc, "mhc_post")
-    return out.reshape(shape)
+    return out
 
 
 def mhc_post_ref(x, h_res, h_out, h_post):

@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .mhc_post import SUPPORTED_N
+from .mhc_post import SUPPORTED_N, _tokens
 
 
 def _flatten(grad_y, x, h_res, h_out, h_post):
@@ -63,24 +63,30 @@ def post_backward_sum_fused(T: int, N: int, D: int, dtype: torch.dtype) -> bool:
 
 def _post_backward(what, grad_y, grad_y2, x, h_res, h_out, h_post):
     _lib.require_device(what, grad_y, x, h_res, h_out, h_post, grad_y2)
-    gy, xf, hres, hout, hpost, shape4, shape_out = _flatten(grad_y, x, h_res, h_out, h_post)
-    T, N, D = gy.shape
+    if grad_y.dim() not in (3, 4):
+        raise ValueError(f"unsupported grad_y.dim()={grad_y.dim()}")
+    T, N, D = _tokens(grad_y)
+    lead = tuple(grad_y.shape[:-2])
+    dt = x.dtype
+    # grad_y and x flatten to the same (T, N, D): any strides of either
+    xf = _lib.operand(x, (T, N, D), dt)
+    gy = _lib.operand(grad_y, (T, N, D), dt)
+    gy2 = None if grad_y2 is None else _lib.operand(grad_y2, (T, N, D), dt)
+    hres_k = _lib.operand(h_res, (T, N, N), torch.float32)
+    hout_k = _lib.operand(h_out, (T, D), dt)
+    hpost_k = _lib.operand(h_post, (T, N), torch.float32)
     if N not in SUPPORTED_N:
         raise NotImplementedError(f"{what}: N={N} not supported (supported: {SUPPORTED_N})")
-    code = _lib.dtype_code(what, xf.dtype)
-    gy = gy.to(xf.dtype).contiguous()
-    gy2 = None if grad_y2 is None else grad_y2.reshape(T, N, D).to(xf.dtype).contiguous()
-    hout_k = hout.to(xf.dtype).contiguous()
-    hres_k = hres.to(torch.float32).contiguous()
-    hpost_k = hpost.to(torch.float32).contiguous()
+    code = _lib.dtype_code(what, dt)
 
-    grad_x = torch.empty_like(xf)
-    grad_hout = torch.empty((T, D), dtype=xf.dtype, device=xf.device)
-    grad_hres = torch.empty((T, N, N), dtype=torch.float32, device=xf.device)
-    grad_hpost = torch.empty((T, N), dtype=torch.float32, device=xf.device)
+    dev = xf.device
+    grad_x = torch.empty(lead + (N, D), dtype=dt, device=dev)
+    grad_hout = torch.empty(lead + (D,), dtype=dt, device=dev)
+    grad_hres = torch.empty(h_res.shape, dtype=torch.float32, device=dev)
+    grad_hpost = torch.empty(h_post.shape, dtype=torch.float32, device=dev)
     if T > 0:
         lib = _lib.load()
-        with torch.cuda.device(xf.device):
+        with _lib.on_device(dev):
             tail = (hres_k.data_ptr(), hout_k.data_ptr(), hpost_k.data_ptr(), grad_x.data_ptr(),
                     grad_hres.data_ptr(), grad_hout.data_ptr(), grad_hpost.data_ptr(), T, N, D, code,
                     _lib.stream_of(xf))
@@ -89,12 +95,7 @@ def _post_backward(what, grad_y, grad_y2, x, h_res, h_out, h_post):
             else:
                 rc = lib.mhc_post_bwd_sum(gy.data_ptr(), gy2.data_ptr(), xf.data_ptr(), *tail)
         _lib.check(rc, what)
-    return (
-        grad_x.reshape(shape4),
-        grad_hres.to(h_res.dtype).reshape(h_res.shape),
-        grad_hout.to(h_out.dtype).reshape(shape_out),
-        grad_hpost.to(h_post.dtype).reshape(h_post.shape),
-    )
+    return (grad_x, grad_hres.to(h_res.dtype), grad_hout.to(h_out.dtype), grad_hpost.to(h_post.dtype))
 
 
 def mhc_post_backward_ref(grad_y, x, h_res, h_out, h_post):

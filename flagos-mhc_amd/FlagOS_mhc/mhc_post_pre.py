@@ -27,7 +27,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .mhc_post import _flatten_bsn
+from .mhc_post import _tokens
 from .mhc_pre_clamp_sinkhorn import SINGLE_PASS_MIN_T, _check_params
 
 
@@ -50,22 +50,22 @@ def mhc_post_pre_clamp_sinkhorn(
     mhc_pre_clamp_sinkhorn(x_next, phi, alpha, base, ...)."""
     _lib.require_device("mhc_post_pre_clamp_sinkhorn", x, h_res, h_out, h_post, phi, alpha, base)
     _lib.SINGLE_PASS.check(block=False)  # earlier calls' bounded waits, where finished
-    xf, hres, hout, hpost, shape = _flatten_bsn(x, h_res, h_out, h_post)
-    T, N, D = xf.shape
+    T, N, D = _tokens(x)
+    xf = x.contiguous()
+    hres = _lib.operand(h_res, (T, N, N), torch.float32)
+    hout = _lib.operand(h_out, (T, D), xf.dtype)
+    hpost = _lib.operand(h_post, (T, N), torch.float32)
     M = _check_params(N, D, phi, alpha, base)
     xcode = _lib.dtype_code("mhc_post_pre_clamp_sinkhorn", xf.dtype)
     phi_c = phi.contiguous()
     pcode = _lib.dtype_code("mhc_post_pre_clamp_sinkhorn (phi)", phi_c.dtype)
-    hres = hres.to(torch.float32).contiguous()
-    hpost = hpost.to(torch.float32).contiguous()
-    hout = hout.to(xf.dtype).contiguous()
-    alpha_c = alpha.reshape(3).to(torch.float32).contiguous()
-    base_c = base.reshape(M).to(torch.float32).contiguous()
+    alpha_c = _lib.operand(alpha, (3,), torch.float32)
+    base_c = _lib.operand(base, (M,), torch.float32)
     dev = xf.device
     f32 = dict(dtype=torch.float32, device=dev)
 
-    x_next = torch.empty_like(xf)
-    y = torch.empty((T, D), dtype=xf.dtype, device=dev)
+    x_next = torch.empty_like(xf, memory_format=torch.contiguous_format)
+    y = torch.empty(tuple(x.shape[:-2]) + (D,), dtype=xf.dtype, device=dev)
     post_out = torch.empty((T, N), **f32)
     comb = torch.empty((T, N, N), **f32)
     inv_rms = mixes = logits = pre = None
@@ -77,15 +77,15 @@ def mhc_post_pre_clamp_sinkhorn(
     if T > 0:
         lib = _lib.load()
         # x that is not bf16 runs the general form, whose workspace is that of an fp32 phi
-        ws_bytes = int(lib.mhc_post_pre_fwd_workspace_size(T, N, D, pcode if xf.dtype == torch.bfloat16 else 0))
-        ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
+        ws, ws_bytes = _lib.workspace("mhc_post_pre_fwd_workspace_size", dev, T, N, D,
+                                      pcode if xf.dtype == torch.bfloat16 else 0)
         # the shapes a single pass can take report its bounded waits into a
         # status word, as the pre forward's
         slot = status = None
         if (N == 4 and T >= SINGLE_PASS_MIN_T and xf.dtype == torch.bfloat16
                 and phi_c.dtype == torch.bfloat16 and not torch.cuda.is_current_stream_capturing()):
             slot, status = _lib.SINGLE_PASS.acquire()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.mhc_post_pre_fwd_ex(
                 xf.data_ptr(), hres.data_ptr(), hout.data_ptr(), hpost.data_ptr(), xcode,
                 phi_c.data_ptr(), pcode, alpha_c.data_ptr(), base_c.data_ptr(), float(norm_eps),
@@ -96,9 +96,8 @@ def mhc_post_pre_clamp_sinkhorn(
         _lib.check(rc, "mhc_post_pre_clamp_sinkhorn")
         if slot is not None:
             _lib.SINGLE_PASS.commit(slot, torch.cuda.current_stream(dev))
-    yshape = shape[:-2] + (D,)
-    out = {"y": y.reshape(yshape), "post_out": post_out, "comb_frag": comb}
+    out = {"y": y, "post_out": post_out, "comb_frag": comb}
     if need_backward:
         out.update(inv_rms=inv_rms, x_scaled=None, mixes=mixes, h_res_logits=logits, pre=pre)
-    return x_next.reshape(shape), out
+    return x_next, out
 

@@ -25,6 +25,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from .mhc_post import _tokens
 
 SUPPORTED_N = (4, 8)
 SINGLE_PASS_MIN_T = 8192  # fewest tokens the single-pass forms take (csrc/pre_fwd_coop.hpp, pre_bwd_coop.hpp)
@@ -55,18 +56,18 @@ def _pre_forward(x, phi, alpha, base, norm_eps, hc_eps, clamp_min, clamp_max, it
                  need_backward, want_x_scaled):
     _lib.require_device("mhc_pre_clamp_sinkhorn", x, phi, alpha, base)
     _lib.SINGLE_PASS.check(block=False)  # earlier calls' bounded waits, where finished
-    xf, yshape = _flatten(x)
-    T, N, D = xf.shape
+    T, N, D = _tokens(x)
+    xf = x.contiguous()
     M = _check_params(N, D, phi, alpha, base)
     xcode = _lib.dtype_code("mhc_pre_clamp_sinkhorn", xf.dtype)
     phi_c = phi.contiguous()
     pcode = _lib.dtype_code("mhc_pre_clamp_sinkhorn (phi)", phi_c.dtype)
-    alpha_c = alpha.reshape(3).to(torch.float32).contiguous()
-    base_c = base.reshape(M).to(torch.float32).contiguous()
+    alpha_c = _lib.operand(alpha, (3,), torch.float32)
+    base_c = _lib.operand(base, (M,), torch.float32)
     dev = xf.device
     f32 = dict(dtype=torch.float32, device=dev)
 
-    y = torch.empty((T, D), dtype=xf.dtype, device=dev)
+    y = torch.empty(tuple(x.shape[:-2]) + (D,), dtype=xf.dtype, device=dev)
     post_out = torch.empty((T, N), **f32)
     comb = torch.empty((T, N, N), **f32)
     inv_rms = mixes = logits = pre = x_scaled = None
@@ -80,8 +81,8 @@ def _pre_forward(x, phi, alpha, base, norm_eps, hc_eps, clamp_min, clamp_max, it
     if T > 0:
         lib = _lib.load()
         # x that is not bf16 runs the general form, whose workspace is that of an fp32 phi
-        ws_bytes = int(lib.mhc_pre_fwd_workspace_size(T, N, D, pcode if xf.dtype == torch.bfloat16 else 0))
-        ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
+        ws, ws_bytes = _lib.workspace("mhc_pre_fwd_workspace_size", dev, T, N, D,
+                                      pcode if xf.dtype == torch.bfloat16 else 0)
         # the shapes the single-pass form can take (N = 4, bf16, T >= 8192;
         # never under stream capture) report its bounded waits into a status word
         slot = status = None
@@ -89,7 +90,7 @@ def _pre_forward(x, phi, alpha, base, norm_eps, hc_eps, clamp_min, clamp_max, it
                 and phi_c.dtype == torch.bfloat16 and not torch.cuda.is_current_stream_capturing()):
             slot, status = _lib.SINGLE_PASS.acquire()
         stream = _lib.stream_of(xf)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.mhc_pre_fwd_ex(
                 xf.data_ptr(), xcode, phi_c.data_ptr(), pcode, alpha_c.data_ptr(),
                 base_c.data_ptr(), float(norm_eps), float(hc_eps), float(clamp_min),
@@ -100,7 +101,7 @@ def _pre_forward(x, phi, alpha, base, norm_eps, hc_eps, clamp_min, clamp_max, it
         _lib.check(rc, "mhc_pre_clamp_sinkhorn")
         if slot is not None:
             _lib.SINGLE_PASS.commit(slot, torch.cuda.current_stream(dev))
-    result = {"y": y.reshape(yshape), "post_out": post_out, "comb_frag": comb}
+    result = {"y": y, "post_out": post_out, "comb_frag": comb}
     if need_backward:
         result.update(inv_rms=inv_rms, x_scaled=x_scaled, mixes=mixes, h_res_logits=logits,
                       pre=pre)

@@ -30,7 +30,8 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .mhc_pre_clamp_sinkhorn import SINGLE_PASS_MIN_T, SUPPORTED_N, _flatten
+from .mhc_post import _tokens
+from .mhc_pre_clamp_sinkhorn import SINGLE_PASS_MIN_T, SUPPORTED_N
 
 
 def mhc_pre_clamp_sinkhorn_backward(
@@ -82,8 +83,8 @@ def _pre_backward(x, phi, alpha, base, inv_rms, mixes, pre, grad_y, grad_post_ou
     if x.dim() not in (3, 4):
         raise ValueError(f"unsupported x.dim()={x.dim()}")
     shape = tuple(x.shape)
-    xf, _ = _flatten(x)
-    T, N, D = xf.shape
+    T, N, D = _tokens(x)
+    xf = x.contiguous()
     if grad_y.dim() == 3:
         _B, _S, _D = grad_y.shape
         assert _B * _S == T and _D == D
@@ -100,27 +101,26 @@ def _pre_backward(x, phi, alpha, base, inv_rms, mixes, pre, grad_y, grad_post_ou
     dev = xf.device
     f32 = dict(dtype=torch.float32, device=dev)
 
-    gy = grad_y.reshape(T, D).to(xf.dtype).contiguous()
-    gpost = grad_post_out.reshape(T, N).to(torch.float32).contiguous()
-    gcomb = grad_comb_frag.reshape(T, N, N).to(torch.float32).contiguous()
-    inv_c = inv_rms.reshape(T).to(torch.float32).contiguous()
-    mixes_c = mixes.reshape(T, M).to(torch.float32).contiguous()
-    pre_c = pre.reshape(T, N).to(torch.float32).contiguous()
-    alpha_c = alpha.reshape(3).to(torch.float32).contiguous()
-    base_c = base.reshape(M).to(torch.float32).contiguous()
+    gy = _lib.operand(grad_y, (T, D), xf.dtype)
+    gpost = _lib.operand(grad_post_out, (T, N), torch.float32)
+    gcomb = _lib.operand(grad_comb_frag, (T, N, N), torch.float32)
+    inv_c = _lib.operand(inv_rms, (T,), torch.float32)
+    mixes_c = _lib.operand(mixes, (T, M), torch.float32)
+    pre_c = _lib.operand(pre, (T, N), torch.float32)
+    alpha_c = _lib.operand(alpha, (3,), torch.float32)
+    base_c = _lib.operand(base, (M,), torch.float32)
 
-    grad_x = torch.empty((T, N * D), dtype=xf.dtype, device=dev)
+    grad_x = torch.empty(shape, dtype=xf.dtype, device=dev)
     grad_phi = torch.empty((M, N * D), **f32)
     grad_alpha = torch.empty((3,), **f32)
     grad_base = torch.empty((M,), **f32)
     lib = _lib.load()
-    ws_bytes = int(lib.mhc_pre_bwd_workspace_size(T, N, D, pcode, int(iter_times)))
-    ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
+    ws, ws_bytes = _lib.workspace("mhc_pre_bwd_workspace_size", dev, T, N, D, pcode, int(iter_times))
     common = (xf.data_ptr(), xcode, phi_c.data_ptr(), pcode, alpha_c.data_ptr(), base_c.data_ptr(),
               inv_c.data_ptr(), mixes_c.data_ptr(), pre_c.data_ptr(), gy.data_ptr(),
               gpost.data_ptr(), gcomb.data_ptr(), float(hc_eps), float(clamp_min),
               float(clamp_max), int(iter_times))
-    gin = None if grad_x_in is None else grad_x_in.reshape(T, N * D).to(xf.dtype).contiguous()
+    gin = None if grad_x_in is None else _lib.operand(grad_x_in, (T, N * D), xf.dtype)
     flags = _lib.PRE_BWD_COMPENSATED if compensated else 0
     if single_pass is not None:
         flags |= _lib.PRE_BWD_SINGLE_PASS if single_pass else _lib.PRE_BWD_TWO_PASS
@@ -132,14 +132,14 @@ def _pre_backward(x, phi, alpha, base, inv_rms, mixes, pre, grad_y, grad_post_ou
             and phi_c.dtype == torch.bfloat16 and gin is None and not compensated
             and not torch.cuda.is_current_stream_capturing()):
         slot, status = _lib.SINGLE_PASS.acquire()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.mhc_pre_bwd_ex(*common, _lib.ptr(gin), grad_x.data_ptr(), grad_phi.data_ptr(),
                                 grad_alpha.data_ptr(), grad_base.data_ptr(), flags, status,
                                 ws.data_ptr(), ws_bytes, T, N, D, _lib.stream_of(xf))
     _lib.check(rc, "mhc_pre_clamp_sinkhorn_backward")
     if slot is not None:
         _lib.SINGLE_PASS.commit(slot, torch.cuda.current_stream(dev))
-    return grad_x.view(*shape), grad_phi.reshape(phi.shape), grad_alpha, grad_base
+    return grad_x, grad_phi, grad_alpha, grad_base
 
 
 def mhc_pre_clamp_sinkhorn_backward_ref(
