@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kBwdThreads) void pre_bwd_small_kernel(PreBwdSmallA
 // ---------------------------------------------------------------------------
 // Kernel B
 // ---------------------------------------------------------------------------
-constexpr int kStreamTile = 16;  // tokens per tile (MFMA K of the grad_phi product)
+constexpr int kStreamTile = 16;  // tokens per tile (with both planes of g the k of the grad_phi product)
 static_assert(kStreamTile == kBwdTile, "kernel A zero-fills the g tiles of the padding tokens");
 
 struct PreBwdStreamArgs {
@@ -451,13 +451,6 @@ struct PreBwdStreamArgs {
   int64_t T;
   int D;
 };
-
-typedef short short4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ floatx4 mfma16x16x16(const u32x2& a, const u32x2& b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4_t, a),
-                                                  __builtin_bit_cast(short4_t, b), c, 0, 0, 0);
-}
 
 }  // namespace mhc
 
@@ -884,11 +877,11 @@ __global__ __launch_bounds__(64 * DmaCfg<N>::G * H) void pre_bwd_dma_kernel(PreB
         const uint32_t lo = xr[2 * w][c >> 1], hi = xr[2 * w + 1][c >> 1];
         xt[w] = (c & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
       }
+      // both planes of g in one MFMA's k (plane, token): half the instructions
+      // of a 16x16x16 one a plane, at the same issue time each
+      const bf16x8 x2 = as_bf16x8(u32x4{xt[0], xt[1], xt[0], xt[1]});
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        ph[mt][c] = mfma16x16x16(u32x2{gt[mt][0], gt[mt][1]}, xt, ph[mt][c]);
-        ph[mt][c] = mfma16x16x16(u32x2{gt[mt][2], gt[mt][3]}, xt, ph[mt][c]);
-      }
+      for (int mt = 0; mt < MT; ++mt) ph[mt][c] = mfma16x16x32(as_bf16x8(gt[mt]), x2, ph[mt][c]);
     }
     // ---- gs = grad_mixes @ phi, then grad_x ---------------------------------
     floatx4 gs[VC];
