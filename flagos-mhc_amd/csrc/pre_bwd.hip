@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "mhc_launch.hpp"
+#include "phi_transpose.hpp"
 #include "pre_common.hpp"
 #include "pre_host.hpp"
 #include "sinkhorn.hpp"
@@ -94,20 +95,26 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float v) {
 // 8 columns, wave_sum, then the 4 waves in order).
 constexpr int kGpreCols = kBwdThreads * 8;
 
-// Blocks in x: at most kGpreGridT, each looping over the tokens
-// blockIdx.x, blockIdx.x + gridDim.x, ..., so the launch stays far below the
+// Blocks in x: nt, at most kGpreGridT, each looping over the tokens
+// blockIdx.x, blockIdx.x + nt, ... (and after them the blocks that prepare
+// phi^T, which the later kernels need: a launch less), so the launch stays far below the
 // 2^32 work-items of a dispatch at any T.
 constexpr int64_t kGpreGridT = 65536;
 
 template <int N, typename S>
 __global__ __launch_bounds__(kBwdThreads) void pre_bwd_gpre_kernel(const void* xv, const void* gyv, float* part,
-                                                                   int64_t T, int D) {
+                                                                   int64_t T, int D, int nt, PhiTArgs pt) {
+  static_assert(kBwdThreads == kPhiTThreads, "blocks past the tokens' prepare phi^T");
+  if ((int)blockIdx.x >= nt) {
+    if (blockIdx.y == 0) phiT_block(pt, blockIdx.x - nt);
+    return;
+  }
   __shared__ float red[kBwdThreads / kWave][N];
   const S* __restrict__ x = static_cast<const S*>(xv);
   const S* __restrict__ gy = static_cast<const S*>(gyv);
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
   const int64_t d = (int64_t)blockIdx.y * kGpreCols + tid * 8;
-  for (int64_t tok = blockIdx.x; tok < T; tok += gridDim.x) {  // uniform over the block
+  for (int64_t tok = blockIdx.x; tok < T; tok += nt) {  // uniform over the block
     float acc[N];
     float g8[8];
     load8u(gy + tok * D, d, D, g8);
@@ -943,13 +950,20 @@ __global__ __launch_bounds__(64 * DmaCfg<N>::G * H) void pre_bwd_dma_kernel(PreB
 // ---------------------------------------------------------------------------
 // Kernels C: fixed-order reductions
 // ---------------------------------------------------------------------------
-__global__ void sum_splits_kernel(const float* __restrict__ part, float* __restrict__ out,
-                                  int64_t n, int nsplit) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int j = 0; j < nsplit; ++j) s += part[(int64_t)j * n + i];
-    out[i] = s;
+// block b of nb: out[i] = sum over the splits, four at a time (n % 4 == 0)
+__device__ __forceinline__ void sum_splits_block(const float* __restrict__ part, float* __restrict__ out, int64_t n,
+                                                 int nsplit, int64_t b, int64_t nb) {
+  const int64_t n4 = n / 4;
+  const floatx4* p = reinterpret_cast<const floatx4*>(part);
+  for (int64_t i = b * blockDim.x + threadIdx.x; i < n4; i += nb * blockDim.x) {
+    floatx4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int j = 0; j < nsplit; ++j) s += p[(int64_t)j * n4 + i];
+    if ((reinterpret_cast<uintptr_t>(out) & 15u) == 0)
+      reinterpret_cast<floatx4*>(out)[i] = s;
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[4 * i + e] = s[e];
   }
 }
 
@@ -1218,13 +1232,10 @@ __global__ void sum_splits_comp_kernel(const float* __restrict__ part, float* __
 // addition (TwoSum) carried into the compensation.
 // status (may be null): the single-pass kernel's status word; nonzero (a
 // timed-out wait) makes the outputs NaN.
-__global__ __launch_bounds__(256) void sum_rows_kernel(const float* __restrict__ partial,
-                                                       int64_t rows, int C,
-                                                       float* __restrict__ out_alpha,
-                                                       float* __restrict__ out_base, int comp,
-                                                       const uint32_t* status) {
+__device__ __forceinline__ void sum_rows_block(const float* __restrict__ partial, int64_t rows, int C,
+                                               float* __restrict__ out_alpha, float* __restrict__ out_base, int comp,
+                                               const uint32_t* status, int c) {
   __shared__ float red[256], redc[256];
-  const int c = blockIdx.x;
   float s = 0.f, cc = 0.f;
   if (comp) {
     for (int64_t i = threadIdx.x; i < rows; i += 256) neumaier_add(s, cc, partial[i * C + c]);
@@ -1254,6 +1265,24 @@ __global__ __launch_bounds__(256) void sum_rows_kernel(const float* __restrict__
     else
       out_base[c - 3] = red[0];
   }
+}
+
+__global__ __launch_bounds__(256) void sum_rows_kernel(const float* __restrict__ partial, int64_t rows, int C,
+                                                       float* __restrict__ out_alpha, float* __restrict__ out_base,
+                                                       int comp, const uint32_t* status) {
+  sum_rows_block(partial, rows, C, out_alpha, out_base, comp, status, blockIdx.x);
+}
+
+// Both sums in one launch: the first C blocks grad_alpha / grad_base, the
+// others grad_phi.
+__global__ __launch_bounds__(256) void sum_all_kernel(const float* __restrict__ partial, int64_t rows, int C,
+                                                      float* __restrict__ out_alpha, float* __restrict__ out_base,
+                                                      const float* __restrict__ part, float* __restrict__ out,
+                                                      int64_t n, int nsplit) {
+  if ((int)blockIdx.x < C)
+    sum_rows_block(partial, rows, C, out_alpha, out_base, 0, nullptr, blockIdx.x);
+  else
+    sum_splits_block(part, out, n, nsplit, blockIdx.x - C, gridDim.x - C);
 }
 
 }  // namespace mhc
@@ -1425,17 +1454,14 @@ static int launch_comp_gphi(const BwdLayout& lay, const PreBwdSmallArgs& sa, flo
 template <int N, typename S>
 static int reduce_tail(const BwdLayout& lay, const PreBwdSmallArgs& sa, float* gphi_part, int nsplit,
                        uint16_t* gpl, float* grad_phi, float* grad_alpha, float* grad_base, hipStream_t st) {
-  int rc;
   if (sa.comp) {
-    rc = launch_comp_gphi<N, S>(lay, sa, gphi_part, gpl, grad_phi, st);
-  } else {
-    const int64_t n = (int64_t)lay.M * lay.K;
-    hipLaunchKernelGGL(sum_splits_kernel, dim3(reduce_grid(n)), dim3(256), 0, st, gphi_part, grad_phi, n,
-                       nsplit);
-    rc = check_launch("pre_bwd_sum_splits");
+    if (int rc = launch_comp_gphi<N, S>(lay, sa, gphi_part, gpl, grad_phi, st)) return rc;
+    return sum_alpha_base(lay, sa, grad_alpha, grad_base, st);
   }
-  if (rc) return rc;
-  return sum_alpha_base(lay, sa, grad_alpha, grad_base, st);
+  const int64_t n = (int64_t)lay.M * lay.K;
+  hipLaunchKernelGGL(sum_all_kernel, dim3((unsigned)lay.C + reduce_grid(n / 4)), dim3(256), 0, st, sa.partial,
+                     lay.nblkA, lay.C, grad_alpha, grad_base, gphi_part, grad_phi, n, nsplit);
+  return check_launch("pre_bwd_sum");
 }
 
 // Buffer ranges are 32-bit: one tile of x rows (16 * N * D bf16) must fit.
@@ -1568,10 +1594,12 @@ static int launch_pre_bwd_coop(const BwdLayout& lay, PreBwdSmallArgs sa, const P
 }
 
 template <int N, typename S>
-static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwdStreamArgs& sta, float* grad_phi,
+static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwdStreamArgs& sta, const PhiTArgs& pt,
+                          float* grad_phi,
                           float* grad_alpha, float* grad_base, bool vec, const void* gin, uint16_t* gpl, hipStream_t st,
                           char* ws, int sp_mode, int32_t* status_out) {
   const dim3 gA((unsigned)lay.nblkA), bA(kBwdThreads);
+  bool phi_ready = false;
   const bool streaming = vec && std::is_same<S, bf16_t>::value;
   if constexpr (N == 4 && std::is_same<S, bf16_t>::value) {
     // sp_mode: 0 never, 1 from kBcAutoT tokens, 2 from kBcMinT (the layout's
@@ -1579,6 +1607,8 @@ static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwd
     const bool single_pass = sp_mode == 2 || (sp_mode == 1 && sa.T >= kBcAutoT);
     if (single_pass && streaming && !gin && !sa.comp && lay.P == 1 && dma_usable<N>(sta.D)) {
       bool used = false;
+      if (int rc = prepare_phiT_planes(pt, st)) return rc;
+      phi_ready = true;
       const int rc = launch_pre_bwd_coop(lay, sa, sta, grad_phi, grad_alpha, grad_base, ws, status_out, st, &used);
       if (rc || used) return rc;
     }
@@ -1586,7 +1616,9 @@ static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwd
   if (!sa.comp) sa.gm = nullptr;  // only the compensated grad_phi reads fp32 grad_mixes
   sa.scale = nullptr;
   int rc;
-  if (streaming && sa.T >= kGpreDmaMinT) {
+  const bool gpre_dma = streaming && sa.T >= kGpreDmaMinT, gpre_split = !gpre_dma && sa.gpre_part;
+  if (!phi_ready && !gpre_split && (rc = prepare_phiT_planes(pt, st))) return rc;
+  if (gpre_dma) {
     // grad_pre through the LDS-pipelined kernel: one chunk of sums per token
     sa.gpre_part = sa.gpre_buf;
     sa.gpre_chunks = 1;
@@ -1594,10 +1626,11 @@ static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwd
                        0, st, static_cast<const bf16_t*>(sa.x), static_cast<const bf16_t*>(sa.gy), sa.gpre_buf,
                        sa.T, sa.D);
     if ((rc = check_launch("pre_bwd_gpre_dma"))) return rc;
-  } else if (sa.gpre_part) {
-    const dim3 gG((unsigned)(sa.T < kGpreGridT ? sa.T : kGpreGridT), (unsigned)lay.gpre_chunks);
+  } else if (gpre_split) {
+    const int nt = (int)(sa.T < kGpreGridT ? sa.T : kGpreGridT);
+    const dim3 gG((unsigned)(nt + (phi_ready ? 0 : phiT_blocks(pt))), (unsigned)lay.gpre_chunks);
     float* part = const_cast<float*>(sa.gpre_part);
-    hipLaunchKernelGGL((pre_bwd_gpre_kernel<N, S>), gG, bA, 0, st, sa.x, sa.gy, part, sa.T, sa.D);
+    hipLaunchKernelGGL((pre_bwd_gpre_kernel<N, S>), gG, bA, 0, st, sa.x, sa.gy, part, sa.T, sa.D, nt, pt);
     if ((rc = check_launch("pre_bwd_gpre"))) return rc;
   }
   hipLaunchKernelGGL((pre_bwd_small_kernel<N, S>), gA, bA, 0, st, sa);
@@ -1614,15 +1647,15 @@ static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwd
 
 template <typename S>
 static int dispatch_pre_bwd(int N, const BwdLayout& lay, const PreBwdSmallArgs& sa,
-                            const PreBwdStreamArgs& sta, float* gphi,
+                            const PreBwdStreamArgs& sta, const PhiTArgs& pt, float* gphi,
                             float* galpha, float* gbase, bool vec, const void* gin, uint16_t* gpl,
                             hipStream_t st, char* ws, int sp_mode, int32_t* status_out) {
   switch (N) {
     case 4:
-      return launch_pre_bwd<4, S>(lay, sa, sta, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
+      return launch_pre_bwd<4, S>(lay, sa, sta, pt, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
                                   status_out);
     case 8:
-      return launch_pre_bwd<8, S>(lay, sa, sta, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
+      return launch_pre_bwd<8, S>(lay, sa, sta, pt, gphi, galpha, gbase, vec, gin, gpl, st, ws, sp_mode,
                                   status_out);
   }
   return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_bwd: N=%d not supported (4, 8)", N);
@@ -1673,8 +1706,8 @@ static int pre_bwd_entry(const void* x, int32_t x_dtype, const void* phi, int32_
                      workspace_bytes, lay.total);
   char* ws = static_cast<char*>(workspace);
   uint16_t* phiT = reinterpret_cast<uint16_t*>(ws + lay.off_phiT);
-  int rc = prepare_phiT_planes(phi, phi_dtype, M, lay.K, phiT, st);
-  if (rc) return rc;
+  if (phi_dtype < 0 || phi_dtype > 2) return set_error(MHC_ERR_UNSUPPORTED, "phi dtype %d not supported", phi_dtype);
+  const PhiTArgs pt{phi, phi_dtype, M, lay.MP32, lay.P, lay.K, phiT};
 
   PreBwdSmallArgs sa{};
   sa.x = x;
@@ -1728,13 +1761,13 @@ static int pre_bwd_entry(const void* x, int32_t x_dtype, const void* phi, int32_
   const int sp = (flags & MHC_PRE_BWD_TWO_PASS) ? 0 : (flags & MHC_PRE_BWD_SINGLE_PASS) ? 2 : 1;
   switch (x_dtype) {
     case MHC_DTYPE_BF16:
-      return dispatch_pre_bwd<bf16_t>(N, lay, sa, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
+      return dispatch_pre_bwd<bf16_t>(N, lay, sa, sta, pt, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
                                       ws, sp, status);
     case MHC_DTYPE_F16:
-      return dispatch_pre_bwd<f16_t>(N, lay, sa, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
+      return dispatch_pre_bwd<f16_t>(N, lay, sa, sta, pt, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
                                      ws, sp, status);
     case MHC_DTYPE_F32:
-      return dispatch_pre_bwd<float>(N, lay, sa, sta, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
+      return dispatch_pre_bwd<float>(N, lay, sa, sta, pt, grad_phi, grad_alpha, grad_base, vec, grad_x_in, gpl, st,
                                      ws, sp, status);
   }
   return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_bwd: x dtype %d not supported", x_dtype);

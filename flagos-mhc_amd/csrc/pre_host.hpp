@@ -85,8 +85,8 @@ int prepare_phi_planes(const void* phi, int32_t phi_dtype, int M, int64_t K, voi
                        size_t ws_bytes, const uint16_t** planes, int64_t* ld,
                        int64_t* plane_stride, int* nplanes, hipStream_t st);
 
-// Writes phi^T as bf16 planes [P][K][MP32] (zero for m >= M) into `dst`.
-int prepare_phiT_planes(const void* phi, int32_t phi_dtype, int M, int64_t K, uint16_t* dst,
-                        hipStream_t st);
+// Writes phi^T as bf16 planes [P][K][MP] (phi_transpose.hpp).
+struct PhiTArgs;
+int prepare_phiT_planes(const PhiTArgs& a, hipStream_t st);
 
 }  // namespace mhc

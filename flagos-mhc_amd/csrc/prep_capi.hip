@@ -5,6 +5,7 @@
 
 #include "common.hpp"
 #include "mhc_launch.hpp"
+#include "phi_transpose.hpp"
 #include "pre_host.hpp"
 
 namespace mhc {
@@ -43,22 +44,7 @@ __global__ void phi_planes_kernel(const void* phi, uint16_t* out, int M, int64_t
   }
 }
 
-// transposed planes [P][K][MP]: out[p][k][m]
-template <typename S>
-__global__ void phiT_planes_kernel(const void* phi, uint16_t* out, int M, int MP, int64_t K,
-                                   int P) {
-  const int64_t total = K * MP;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t k = i / MP;
-    const int m = (int)(i - k * MP);
-    const float v = m < M ? phi_value<S>(phi, (int64_t)m * K + k) : 0.f;
-    uint32_t hi, lo;
-    split2_bf16(v, hi, lo);
-    out[i] = (uint16_t)hi;
-    if (P > 1) out[total + i] = (uint16_t)lo;
-  }
-}
+__global__ __launch_bounds__(kPhiTThreads) void phiT_planes_kernel(PhiTArgs a) { phiT_block(a, blockIdx.x); }
 
 static unsigned grid_for(int64_t total) {
   int64_t g = (total + 255) / 256;
@@ -105,24 +91,8 @@ int prepare_phi_planes(const void* phi, int32_t phi_dtype, int M, int64_t K, voi
   return check_launch("phi_planes");
 }
 
-int prepare_phiT_planes(const void* phi, int32_t phi_dtype, int M, int64_t K, uint16_t* dst,
-                        hipStream_t st) {
-  const int P = phi_bwd_planes(phi_dtype);
-  const int MP = (int)round_up(M, 32);
-  const int64_t total = K * MP;
-  switch (phi_dtype) {
-    case MHC_DTYPE_BF16:
-      hipLaunchKernelGGL(phiT_planes_kernel<bf16_t>, dim3(grid_for(total)), dim3(256), 0, st, phi, dst, M, MP, K, P);
-      break;
-    case MHC_DTYPE_F16:
-      hipLaunchKernelGGL(phiT_planes_kernel<f16_t>, dim3(grid_for(total)), dim3(256), 0, st, phi, dst, M, MP, K, P);
-      break;
-    case MHC_DTYPE_F32:
-      hipLaunchKernelGGL(phiT_planes_kernel<float>, dim3(grid_for(total)), dim3(256), 0, st, phi, dst, M, MP, K, P);
-      break;
-    default:
-      return set_error(MHC_ERR_UNSUPPORTED, "phi dtype %d not supported", phi_dtype);
-  }
+int prepare_phiT_planes(const PhiTArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(phiT_planes_kernel, dim3((unsigned)phiT_blocks(a)), dim3(kPhiTThreads), 0, st, a);
   return check_launch("phiT_planes");
 }
 
