@@ -34,7 +34,6 @@
 namespace mhc {
 
 constexpr int kFwdTile = 64;  // tokens per block
-constexpr size_t kPreFwdWsBase = 256;  // workspace bytes before the split-K area
 constexpr int kFwdThreads = 256;
 
 struct PreFwdArgs {
@@ -1285,7 +1284,7 @@ extern "C" size_t mhc_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, in
   size_t base = pre_fwd_ws_min(T, N, D, phi_dtype);
   if (N != 4 && N != 8) return base;
   if (phi_dtype != MHC_DTYPE_BF16 || D % 8) {  // the general form's sums
-    const size_t gen = D > 0 && T > 0 ? gen_ws_bytes(T, N, D) : 0;
+    const size_t gen = D > 0 && T > 0 ? gen_ws_bytes(T, N, D, device_cu_count()) : 0;
     return gen > base ? gen : base;
   }
   const size_t coop = coop_ws_bytes(T, N, D);
@@ -1405,7 +1404,7 @@ extern "C" int mhc_pre_fwd_ex(const void* x, int32_t x_dtype, const void* phi, i
   if (x_dtype < 0 || x_dtype > 2) return set_error(MHC_ERR_UNSUPPORTED, "mhc_pre_fwd: x dtype %d not supported", x_dtype);
   if (phi_dtype < 0 || phi_dtype > 2) return set_error(MHC_ERR_UNSUPPORTED, "phi dtype %d not supported", phi_dtype);
   const bool streaming = x_dtype == MHC_DTYPE_BF16 && phi_dtype == MHC_DTYPE_BF16 && vec && K % 8 == 0 && aligned16(phi);
-  const int64_t chunk = streaming || !workspace ? 0 : gen_chunk(T, N, D, workspace_bytes);
+  const int64_t chunk = streaming || !workspace ? 0 : gen_chunk(T, N, D, device_cu_count(), workspace_bytes);
   if (chunk > 0) {
     a.phi_raw = phi;
     return dispatch_pre_fwd_gen(N, x_dtype, a, phi_dtype, chunk, workspace, st);

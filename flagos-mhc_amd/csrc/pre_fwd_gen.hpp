@@ -500,40 +500,9 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_gen_y_kernel(Pre
 // lost as much at wide rows.
 static bool finish_applies(int64_t T, int N, int D) { return T <= 1024 || (D >= 512 && (N == 8 || T <= 2048)); }
 
-constexpr int kGenSmallT = 64;   // tokens up to which the 16-token tiles run
-constexpr int kGenFewUnits = 128;  // .. and stages of 128-token tiles below which they do
-constexpr int kGenMaxSlots = 128;  // slots of a tile's sums, at most about
-
-struct GenPlan {
-  bool small = false;
-  int nst = 0, tt = 0, slots = 0;
-  int64_t w = 0, blocks = 0;
-  size_t bytes = 0;  // sums, pre and inv_rms
-};
-
-static GenPlan gen_plan(int64_t T, int N, int D) {
-  GenPlan p;
-  if (T <= 0) return p;
-  const int M = 2 * N + N * N, cw = N == 8 ? 64 : 128;
-  const int64_t K = (int64_t)N * D;
-  p.small = T <= kGenSmallT || (T + 127) / 128 * ((K + cw - 1) / cw) < kGenFewUnits;
-  const int cws = N == 8 || !p.small ? cw : 256;
-  p.tt = p.small ? 16 : 128;
-  p.nst = (int)((K + cws - 1) / cws);
-  const int64_t total = (T + p.tt - 1) / p.tt * p.nst;
-  const int64_t resident = 2 * (int64_t)device_cu_count();
-  p.w = (total + resident - 1) / resident;
-  if (p.w < (p.nst + kGenMaxSlots - 1) / kGenMaxSlots) p.w = (p.nst + kGenMaxSlots - 1) / kGenMaxSlots;
-  p.blocks = (total + p.w - 1) / p.w;
-  p.slots = (int)((p.nst + p.w - 1) / p.w) + 1;
-  if (p.slots > p.blocks) p.slots = (int)p.blocks;
-  p.bytes = align256((size_t)p.slots * T * M * 4) + align256((size_t)p.slots * T * 4) + fwd_y_ws_bytes(T, N);
-  return p;
-}
-
 template <int N, typename S, typename PT>
 static int launch_gen_contraction(const PreFwdArgs& a, const GenPlan& p, hipStream_t st) {
-  const dim3 grid((unsigned)p.blocks);
+  const dim3 grid((unsigned)p.blocks(a.T));
   if (p.small)
     hipLaunchKernelGGL((pre_fwd_gen_kernel<N, S, PT, true>), grid, dim3(GenCfg<N, true>::THREADS), 0, st, a);
   else
@@ -557,18 +526,14 @@ static int launch_pre_fwd_finish(const PreFwdArgs& a, int nsplit, hipStream_t st
 }
 
 template <int N, typename S>
-static int launch_pre_fwd_gen_chunk(PreFwdArgs a, int32_t phi_dtype, char* w, hipStream_t st) {
-  const GenPlan p = gen_plan(a.T, N, a.D);
-  constexpr int M = 2 * N + N * N;
+static int launch_pre_fwd_gen_chunk(PreFwdArgs a, const GenPlan& p, int32_t phi_dtype, char* w, hipStream_t st) {
   a.gen_nst = p.nst;
   a.gen_w = p.w;
   a.gen_tt = p.tt;
   a.part = reinterpret_cast<float*>(w);
-  w += align256((size_t)p.slots * a.T * M * 4);
-  a.part_ssq = reinterpret_cast<float*>(w);
-  w += align256((size_t)p.slots * a.T * 4);
-  a.pre_ws = reinterpret_cast<float*>(w);
-  a.inv_ws = reinterpret_cast<float*>(w + align256((size_t)a.T * N * 4));
+  a.part_ssq = reinterpret_cast<float*>(w + p.ssq_off);
+  a.pre_ws = reinterpret_cast<float*>(w + p.pre_off);
+  a.inv_ws = reinterpret_cast<float*>(w + p.inv_off);
   int rc = phi_dtype == MHC_DTYPE_BF16  ? launch_gen_contraction<N, S, bf16_t>(a, p, st)
            : phi_dtype == MHC_DTYPE_F16 ? launch_gen_contraction<N, S, f16_t>(a, p, st)
                                         : launch_gen_contraction<N, S, float>(a, p, st);
@@ -588,30 +553,13 @@ static int launch_pre_fwd_gen_chunk(PreFwdArgs a, int32_t phi_dtype, char* w, hi
   return check_launch("pre_fwd_gen_y");
 }
 
-// Tokens a call of the general form takes at a time in `bytes` of workspace:
-// all of them, or a multiple of the tile of at least kGenMinChunk (below that
-// 0: the caller runs the form that needs no sums in memory).
-constexpr int64_t kGenMinChunk = 4096;
-static int64_t gen_chunk(int64_t T, int N, int D, size_t bytes) {
-  if (bytes <= kPreFwdWsBase) return 0;
-  bytes -= kPreFwdWsBase;
-  int64_t c = T;
-  while (gen_plan(c, N, D).bytes > bytes) {
-    c = round_up(c / 2, 128);
-    if (c < kGenMinChunk || c >= T) return 0;
-  }
-  return c;
-}
-
-// Workspace of the general form for all T tokens at once.
-static size_t gen_ws_bytes(int64_t T, int N, int D) { return kPreFwdWsBase + gen_plan(T, N, D).bytes; }
-
-// The general form on `chunk` tokens at a time (the stream orders the chunks'
-// use of the workspace).
+// The general form on `chunk` tokens at a time, all by the plan of a whole
+// chunk (the stream orders the chunks' use of the workspace).
 template <int N, typename S>
 static int launch_pre_fwd_gen(const PreFwdArgs& a, int32_t phi_dtype, int64_t chunk, void* workspace,
                               hipStream_t st) {
   constexpr int M = 2 * N + N * N;
+  const GenPlan p = gen_plan(chunk, N, a.D, device_cu_count());
   for (int64_t t0 = 0; t0 < a.T; t0 += chunk) {
     PreFwdArgs c = a;
     c.T = a.T - t0 < chunk ? a.T - t0 : chunk;
@@ -625,7 +573,7 @@ static int launch_pre_fwd_gen(const PreFwdArgs& a, int32_t phi_dtype, int64_t ch
     if (a.pre) c.pre = a.pre + t0 * N;
     if (a.x_scaled) c.x_scaled = a.x_scaled + t0 * N * a.D;
     const int rc =
-        launch_pre_fwd_gen_chunk<N, S>(c, phi_dtype, static_cast<char*>(workspace) + kPreFwdWsBase, st);
+        launch_pre_fwd_gen_chunk<N, S>(c, p, phi_dtype, static_cast<char*>(workspace) + kPreFwdWsBase, st);
     if (rc) return rc;
   }
   return MHC_OK;

@@ -6,10 +6,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
-namespace mhc {
+#include "pre_fwd_plan.hpp"
 
-inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
-inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
+namespace mhc {
 
 // bf16 planes carrying phi in the forward contraction: 1 for bf16, 2 for fp16
 // (exact), 3 for fp32 (residual below 2^-26, so mixes keep fp32 accuracy).
@@ -73,10 +72,6 @@ int post_pre_fwd_single_pass(const void* x, const float* h_res, const void* h_ou
                              float* post_out, float* comb_frag, float* inv_rms, float* mixes, float* h_res_logits,
                              float* pre, void* workspace, size_t workspace_bytes, int32_t* status, int64_t T,
                              int32_t D, hipStream_t st, bool* used);
-
-// Bytes the pre forward (and the fused post + pre forward) keep per call for
-// pre (T, N) and inv_rms (T,) between their contraction and y kernels.
-inline size_t fwd_y_ws_bytes(int64_t T, int N) { return align256((size_t)T * N * 4) + align256((size_t)T * 4); }
 
 // Makes phi available as bf16 planes [P][M][ld].  bf16 phi with K % 8 == 0
 // and a 16-byte aligned base is used in place; anything else is converted

@@ -123,3 +123,28 @@ def test_workspace_smaller_than_asked(share, T):
     for k in FWD_KEYS:
         assert_close(o[k], want[k].double().cpu().numpy(), 1e-4, 1e-5, k)
     assert_close(o["x_scaled"], want["x_scaled"].double().cpu().numpy().reshape(T, N * D), 1e-5, 1e-6, "x_scaled")
+
+
+@pytest.mark.parametrize("T,N,D,size", [(16512, 4, 256, 4326656), (8297, 4, 512, 3900000), (11826, 8, 82, 13861120)])
+def test_chunks_write_inside_the_workspace(T, N, D, size):
+    """Chunks whose last, shorter piece would by a plan of its own take more
+    slots than a whole one: the bytes behind the workspace stay as they are,
+    and every output is that of the call with the full workspace, to rounding."""
+    print(f"[pre_fwd general] guarded workspace T={T} N={N} D={D} {size}", flush=True)
+    x, phi, alpha, base, *_ = pre_inputs(T, N, D, BF, F32, seed=D)
+    lib = _lib.load()
+    full, guard = lib.mhc_pre_fwd_workspace_size(T, N, D, 0), 16 << 20
+    assert size < full < size + guard
+    want = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, **_kw())
+    ws = torch.full((size + guard,), 0x5a, dtype=torch.uint8, device=DEV)
+    y, post = torch.empty(T, D, device=DEV, dtype=BF), torch.empty(T, N, device=DEV, dtype=F32)
+    comb = torch.empty(T, N, N, device=DEV, dtype=F32)
+    rc = lib.mhc_pre_fwd(x.data_ptr(), 1, phi.data_ptr(), 0, alpha.data_ptr(), base.data_ptr(), 1e-6, 1e-6, -10.0,
+                         10.0, 20, y.data_ptr(), post.data_ptr(), comb.data_ptr(), None, None, None, None, None,
+                         ws.data_ptr(), size, T, N, D, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "mhc_pre_fwd")
+    torch.cuda.synchronize()
+    assert bool((ws[size:] == 0x5a).all())
+    assert_close(y, want["y"].double().cpu().numpy(), 2e-2, 2e-2, "y")
+    assert_close(post, want["post_out"].double().cpu().numpy(), 1e-4, 1e-5, "post_out")
+    assert_close(comb, want["comb_frag"].double().cpu().numpy(), 1e-4, 1e-5, "comb_frag")
