@@ -76,9 +76,8 @@ def mhc_post_pre_clamp_sinkhorn(
         pre = torch.empty((T, N), **f32)
     if T > 0:
         lib = _lib.load()
-        # x that is not bf16 runs the general form, whose workspace is that of an fp32 phi
         ws, ws_bytes = _lib.workspace("mhc_post_pre_fwd_workspace_size", dev, T, N, D,
-                                      pcode if xf.dtype == torch.bfloat16 else 0)
+                                      _lib.pre_fwd_size_code(pcode, phi_c, x_next))
         # the shapes a single pass can take report its bounded waits into a
         # status word, as the pre forward's
         slot = status = None

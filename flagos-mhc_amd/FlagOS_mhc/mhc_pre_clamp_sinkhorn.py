@@ -80,9 +80,8 @@ def _pre_forward(x, phi, alpha, base, norm_eps, hc_eps, clamp_min, clamp_max, it
             x_scaled = torch.empty((T, N * D), **f32)
     if T > 0:
         lib = _lib.load()
-        # x that is not bf16 runs the general form, whose workspace is that of an fp32 phi
         ws, ws_bytes = _lib.workspace("mhc_pre_fwd_workspace_size", dev, T, N, D,
-                                      pcode if xf.dtype == torch.bfloat16 else 0)
+                                      _lib.pre_fwd_size_code(pcode, phi_c, xf))
         # the shapes the single-pass form can take (N = 4, bf16, T >= 8192;
         # never under stream capture) report its bounded waits into a status word
         slot = status = None

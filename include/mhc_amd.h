@@ -110,7 +110,9 @@ int mhc_post_bwd_sum_fused(int64_t T, int32_t N, int32_t D, int32_t dtype);
  * general form's sums over split columns (at most ~128 * 25 floats a token at
  * few tokens, ~3 * 25 from 16384 on); with less, the tokens run in chunks that
  * fit, or in a slower form that needs only phi's bf16 planes.  x that is not
- * bf16 runs the general form whatever phi is: ask with MHC_DTYPE_F32 then.
+ * bf16, and x, phi, y or x_scaled that is not 16-byte aligned, run the general
+ * form whatever phi is: ask with MHC_DTYPE_F32 then (less may be refused where
+ * it does not hold phi's planes either).
  */
 size_t mhc_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, int32_t phi_dtype);
 int mhc_pre_fwd(const void* x, int32_t x_dtype, const void* phi, int32_t phi_dtype,

@@ -148,3 +148,34 @@ def test_chunks_write_inside_the_workspace(T, N, D, size):
     assert_close(y, want["y"].double().cpu().numpy(), 2e-2, 2e-2, "y")
     assert_close(post, want["post_out"].double().cpu().numpy(), 1e-4, 1e-5, "post_out")
     assert_close(comb, want["comb_frag"].double().cpu().numpy(), 1e-4, 1e-5, "comb_frag")
+
+
+@pytest.mark.parametrize("which", ["x", "phi", "both"])
+@pytest.mark.parametrize("T,D", [(1, 7168), (40, 1024), (8200, 520), (16157, 1040)])
+def test_unaligned_bf16_calls_get_the_general_workspace(T, D, which):
+    """bf16 x and phi one element into their storage, few tokens and many:
+    such a call runs the general form and needs its workspace (a phi that is
+    not aligned was refused at few tokens, its planes not fitting)."""
+    N = 4
+    print(f"[pre_fwd general] unaligned bf16 {which} T={T} D={D}", flush=True)
+    x, phi, alpha, base, *_ = pre_inputs(T, N, D, BF, BF, seed=T)
+    want = m.mhc_pre_clamp_sinkhorn(x, phi, alpha, base, **_kw())
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, device=DEV, dtype=t.dtype)
+        buf[1:] = t.reshape(-1)
+        return buf[1:].view(t.shape)
+
+    xs, ps = (shifted(x) if which != "phi" else x), (shifted(phi) if which != "x" else phi)
+    assert _lib.pre_fwd_size_code(1, ps, xs) == 0 and _lib.pre_fwd_size_code(1, phi, x) == 1
+    out = m.mhc_pre_clamp_sinkhorn(xs, ps, alpha, base, **_kw())
+    h_res, h_post = want["comb_frag"], want["post_out"]
+    h_out = x[:, 0].contiguous()
+    x_next, fused = m.mhc_post_pre_clamp_sinkhorn(xs, h_res, h_out, h_post, ps, alpha, base, **_kw())
+    x_want, fused_want = m.mhc_post_pre_clamp_sinkhorn(x, h_res, h_out, h_post, phi, alpha, base, **_kw())
+    torch.cuda.synchronize()
+    assert torch.equal(x_next, x_want)
+    for got, ref in ((out, want), (fused, fused_want)):
+        assert_close(got["y"], ref["y"].double().cpu().numpy(), 2e-2, 2e-2, "y")
+        for k in ("post_out", "comb_frag"):
+            assert_close(got[k], ref[k].double().cpu().numpy(), 1e-4, 1e-5, k)
