@@ -30,7 +30,10 @@
 // few loads; the waves' sums meet in LDS at the end of a tile's run.
 //
 // A stage's products go through a fresh MFMA chain that is added to the
-// running sums by round-to-nearest adds (a chain over all of K drifts).
+// running sums by round-to-nearest adds (a chain over all of K drifts), and a
+// stage's squares through a chain of their own: one over a block's whole run
+// loses the small squares, which all round the same way (inv_rms at T = 65536,
+// D = 7168, bf16: 3.1e-6 off so, 7e-8 now, at the same time).
 //
 // Measured (MI355X, the whole operator; before: one block a 64-token tile
 // that walked all of K with one wave a SIMD, then y): phi fp32, bf16 x, N =
@@ -259,6 +262,7 @@ __global__ __launch_bounds__((GenCfg<N, SMALL>::THREADS), (gen_min_waves<N, S, P
 
   auto compute = [&](const Raw8<S>(&X)[STEPS], int buf) {
     floatx4 part[MT];
+    float sq = 0.f;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) part[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -269,7 +273,7 @@ __global__ __launch_bounds__((GenCfg<N, SMALL>::THREADS), (gen_min_waves<N, S, P
       gen_unpack(X[i], f);
       gen_planes(X[i], f, xp);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ssq = fmaf(f[e], f[e], ssq);
+      for (int e = 0; e < 8; ++e) sq = fmaf(f[e], f[e], sq);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -283,6 +287,7 @@ __global__ __launch_bounds__((GenCfg<N, SMALL>::THREADS), (gen_min_waves<N, S, P
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] += part[mt];
+    ssq += sq;
   };
 
   // the block's sums of a tile: lane (r, q) of acc[mt] holds token 16 wt +

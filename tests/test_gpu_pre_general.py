@@ -11,6 +11,7 @@ import torch
 
 import FlagOS_mhc as m
 from FlagOS_mhc import _lib
+from FlagOS_mhc.mhc_pre_clamp_sinkhorn import _pre_forward
 from test_gpu_post import DEV, _subset, assert_close
 from test_gpu_pre import FWD_KEYS, _oracle_fwd, check_fwd, pre_inputs
 
@@ -179,3 +180,19 @@ def test_unaligned_bf16_calls_get_the_general_workspace(T, D, which):
         assert_close(got["y"], ref["y"].double().cpu().numpy(), 2e-2, 2e-2, "y")
         for k in ("post_out", "comb_frag"):
             assert_close(got[k], ref[k].double().cpu().numpy(), 1e-4, 1e-5, k)
+
+
+@pytest.mark.parametrize("T,N,D,dtype", [(65536, 4, 4096, BF), (65536, 8, 1031, BF), (32768, 4, 4096, HF)])
+def test_inv_rms_of_long_runs(T, N, D, dtype):
+    """Many tokens, so that a block sums most of a row by itself: inv_rms keeps
+    fp32 accuracy.  A lane adds at most 260 stages' squares (32 or 16 each, in
+    chains of their own) to its quarter of the row; 260 roundings of at most
+    2^-24 of the running sum, at random, are below sqrt(260 / 3) 2^-24 = 5.6e-7
+    of it, four quarters and the square root take that to 1.4e-7, and inv_rms
+    itself is rounded (2^-24): 3e-7 in 2-norm (one chain over the run:
+    1e-6 to 3e-6)."""
+    print(f"[pre_fwd general] inv_rms T={T} N={N} D={D} {dtype}", flush=True)
+    x, phi, alpha, base, *_ = pre_inputs(T, N, D, dtype, F32, seed=7)
+    got = _pre_forward(x, phi, alpha, base, 1e-6, 1e-6, -10.0, 10.0, 20, True, False)["inv_rms"]
+    want = torch.cat([torch.rsqrt(c.double().reshape(len(c), -1).square().mean(1) + 1e-6) for c in x.split(4096)])
+    assert float((got.double() - want).norm() / want.norm()) < 3e-7
