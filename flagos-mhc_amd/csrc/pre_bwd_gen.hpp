@@ -21,8 +21,14 @@
 //     the tokens and columns that it loaded, so
 //     grad_x = grad_y pre + inv gs + scale x (+ grad_x_in) is formed and
 //     stored in place.
-// No LDS and no barriers: a wave waits for nothing but its own loads.  It
-// replaces a kernel that staged 32 tokens x 256 columns in LDS (element by
+// gs comes first: its operands arrive first, and grad_phi's conversions of x
+// then run between MFMAs (N = 8, one wave a SIMD, T = 8192, D = 1024 fp16: 193
+// us the other way round, 164 so; N = 4 equal).
+// grad_phi is added in MFMA chains of 64 tiles, which meet in fp32 sums in
+// LDS by round-to-nearest adds: one chain over a block's tiles drifts with
+// their number (2-norm error against 64 bits, bf16, one chain / so: N = 8, D =
+// 8191, T = 32768 4.2e-6 / 2.5e-6; N = 4, D = 8191, T = 65536 4.1e-6 / 2.5e-6).
+// No barriers: a wave waits for nothing but its own loads.  It replaces a kernel that staged 32 tokens x 256 columns in LDS (element by
 // element for unaligned rows) between barriers.  Measured, whole backward on
 // MI355X, before -> after: fp16, N = 4, T = 8192: D = 1003 291 -> 115 us, D =
 // 1024 145 -> 80; bf16 T = 16384, D = 907 510 -> 174; fp32 T = 8192, D = 2048
@@ -45,6 +51,8 @@ template <int N, typename S> struct GenBwdCfg {
   static constexpr int BLOCKS_PER_CU = N == 4 ? 2 : 1;
   static_assert(NW == 2 || NW == 4, "8- or 16-byte row pieces");
 };
+
+constexpr int kGenBwdStretch = 64;  // tiles of an MFMA chain of grad_phi
 
 template <int NW> struct GenWords { uint32_t w[NW]; };
 
@@ -134,11 +142,29 @@ __global__ __launch_bounds__((GenBwdCfg<N, S>::THREADS), (GenBwdCfg<N, S>::BLOCK
       for (int p = 0; p < P; ++p)
         pb[c][mk][p] = ld16(a.phiT + p * a.phiT_plane_stride + (kc + c) * MP32 + 32 * mk + 8 * q);
 
+  // grad_phi: the tiles of a stretch in ph, those of the stretches before in
+  // LDS (a lane's own sums; N = 4 has no registers for them)
+  __shared__ floatx4 run[MT * VC][C::THREADS];
+  const bool folds = ntiles > (int64_t)kGenBwdStretch * nsplit;
   floatx4 ph[MT][VC];
+  auto clear = [&]() {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int c = 0; c < VC; ++c) ph[mt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < VC; ++c) ph[mt][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < MT * VC; ++i) {
+      run[i][threadIdx.x] += ph[i / VC][i % VC];
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // not all of them in registers at once
+    }
+  };
+  clear();
+  if (folds) {
+#pragma unroll
+    for (int i = 0; i < MT * VC; ++i) run[i][threadIdx.x] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // Rows past T read row T - 1: its x meets zero columns of g (kernel A
   // zero-fills the padding tokens of the last tile) and its grad_x is not
@@ -154,9 +180,10 @@ __global__ __launch_bounds__((GenBwdCfg<N, S>::THREADS), (GenBwdCfg<N, S>::BLOCK
     }
   };
 
-  Row xr[4], gr[4], xn[4], gn[4];
+  Row xn[4], gn[4];
   if (split < ntiles) load_rows(split, xn, gn);
-  for (int64_t tile = split; tile < ntiles; tile += nsplit) {
+  auto step = [&](int64_t tile) {
+    Row xr[4], gr[4];
     const int64_t tb = tile * TT;
     // ---- operands of the tile (L2), then the next tile's rows --------------
     float4 cf[4];
@@ -197,6 +224,18 @@ __global__ __launch_bounds__((GenBwdCfg<N, S>::THREADS), (GenBwdCfg<N, S>::BLOCK
         for (int e = 0; e < 4; ++e) gen_join<S, NW>(gr[e], gj[e], VC - cb);
       }
     }
+    // ---- gs = grad_mixes phi, then grad_x -----------------------------------
+    floatx4 gs[VC];
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      gs[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int mk = 0; mk < MK; ++mk) {
+        gs[c] = mfma16x16x32(as_bf16x8(gA[mk][0]), as_bf16x8(pb[c][mk][0]), gs[c]);
+        gs[c] = mfma16x16x32(as_bf16x8(gA[mk][1]), as_bf16x8(pb[c][mk][0]), gs[c]);
+        if constexpr (P > 1) gs[c] = mfma16x16x32(as_bf16x8(gA[mk][0]), as_bf16x8(pb[c][mk][P - 1]), gs[c]);
+      }
+    }
     // ---- grad_phi partial += g^T x over the tile's 16 tokens --------------
 #pragma unroll
     for (int c = 0; c < VC; ++c) {
@@ -219,18 +258,6 @@ __global__ __launch_bounds__((GenBwdCfg<N, S>::THREADS), (GenBwdCfg<N, S>::BLOCK
         bx[p][3] = bx[p][1];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) ph[mt][c] = mfma16x16x32(as_bf16x8(ga[mt]), as_bf16x8(bx[p]), ph[mt][c]);
-      }
-    }
-    // ---- gs = grad_mixes phi, then grad_x -----------------------------------
-    floatx4 gs[VC];
-#pragma unroll
-    for (int c = 0; c < VC; ++c) {
-      gs[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int mk = 0; mk < MK; ++mk) {
-        gs[c] = mfma16x16x32(as_bf16x8(gA[mk][0]), as_bf16x8(pb[c][mk][0]), gs[c]);
-        gs[c] = mfma16x16x32(as_bf16x8(gA[mk][1]), as_bf16x8(pb[c][mk][0]), gs[c]);
-        if constexpr (P > 1) gs[c] = mfma16x16x32(as_bf16x8(gA[mk][0]), as_bf16x8(pb[c][mk][P - 1]), gs[c]);
       }
     }
 #pragma unroll
@@ -263,6 +290,33 @@ __global__ __launch_bounds__((GenBwdCfg<N, S>::THREADS), (GenBwdCfg<N, S>::BLOCK
         __builtin_nontemporal_store(v, reinterpret_cast<u32x2_a2*>(row));
       }
     }
+  };
+  // One loop at N = 4 (two take 20 registers more, and rows of fp32 then
+  // spill); two at N = 8, whose accumulators are AGPRs: folded inside the loop
+  // over tiles they, or phi^T, move between register files at every tile.
+  if constexpr (N == 4) {
+    int done = 0;
+    for (int64_t tile = split; tile < ntiles; tile += nsplit) {
+      step(tile);
+      if (folds && ++done == kGenBwdStretch) {
+        done = 0;
+        fold();
+        clear();
+      }
+    }
+  } else {
+    const int64_t span = (int64_t)kGenBwdStretch * nsplit;
+    int64_t tile = split;
+    while (folds && tile + span < ntiles) {
+      for (const int64_t end = tile + span; tile < end; tile += nsplit) step(tile);
+      fold();
+      clear();
+    }
+    for (; tile < ntiles; tile += nsplit) step(tile);
+  }
+  if (folds) {
+#pragma unroll
+    for (int i = 0; i < MT * VC; ++i) ph[i / VC][i % VC] += run[i][threadIdx.x];
   }
 
   float* part = a.gphi_part + (int64_t)split * M * K + kl;

@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import FlagOS_mhc as m
+from FlagOS_mhc.mhc_pre_clamp_sinkhorn import _pre_forward
 from FlagOS_mhc.mhc_pre_clamp_sinkhorn_backward import _pre_backward
 from gpu_ref import check_reductions, pre_bwd_fp64
 from oracle import mhc_oracle as orc
@@ -74,3 +75,19 @@ def test_unaligned_bases_and_grad_x_in(T, N, D, dtype, phi_dtype):
     _check(T, N, D, dtype, phi_dtype, "unaligned", shift=True)
     _check(T, N, D, dtype, phi_dtype, "unaligned, grad_x_in", shift=True, gin=True)
     _check(T, N, D, dtype, phi_dtype, "grad_x_in", gin=True)
+
+
+@pytest.mark.parametrize("T,N,D,dtype", [(32768, 8, 4100, BF), (32768, 4, 8190, BF)])
+def test_grad_phi_of_long_chains(T, N, D, dtype):
+    """Wide rows and many tokens: few token splits, a block walks 680 or 2048
+    tiles.  bf16 x is exact; the two bf16 planes of g leave at most 2^-18 of
+    each term, at random, 2^-18 / sqrt(3) = 2.2e-6 of the sum in 2-norm; fp32
+    sums and the forward's mixes add some 1e-7 (one MFMA chain over a block's
+    tiles: 3.2e-6 and 3.4e-6)."""
+    print(f"[pre_bwd general] grad_phi chains T={T} N={N} D={D} {dtype}", flush=True)
+    x, phi, alpha, base, gy, gpost, gcomb = pre_inputs(T, N, D, dtype, dtype, seed=1)
+    out = _pre_forward(x, phi, alpha, base, 1e-6, 1e-6, -10.0, 10.0, 20, True, False)
+    gphi = _pre_backward(x, phi, alpha, base, out["inv_rms"], out["mixes"], out["pre"], gy, gpost, gcomb,
+                         1e-6, 1e-6, -10.0, 10.0, 20)[1]
+    want = pre_bwd_fp64(x, phi, alpha, base, gy, gpost, gcomb, KW)["grad_phi"]
+    assert float((gphi.double().reshape(want.shape) - want).norm() / want.norm()) < 2.7e-6
