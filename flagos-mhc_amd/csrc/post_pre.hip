@@ -64,14 +64,11 @@ namespace mhc {
 
 namespace {
 
-constexpr int kPPN = 4;
-constexpr int kPPM = 2 * kPPN + kPPN * kPPN;  // 24
+// kPPN, kPPM, kPPTile and kPPCW: pre_fwd_plan.hpp
 constexpr int kPPMT = 2;                      // 16-row m tiles (rows >= 24 load as zero)
-constexpr int kPPTile = 32;                   // tokens per tile
 constexpr int kPPWaves = 8;
 constexpr int kPPThreads = kPPWaves * kWave;
 constexpr int kPPStages = 4;                  // ring slots
-constexpr int kPPCW = 64;                     // d columns per contraction stage
 constexpr int kUH = 16, kUP = 20;             // first h_out / phi unit of a contraction slot
 constexpr int kPPUnits = 36;                  // 1 KB units per slot
 constexpr int kPPCImax = (kPPUnits + kPPWaves - 1) / kPPWaves;  // 5: loads of waves 0..3
@@ -100,8 +97,8 @@ struct PostPreArgs {
   float* pre;
   float* pre_ws;         // (T, 4) pre for the y kernel
   // otherwise
-  float* part;           // [slot][T][M] sums of x_next . phi^T over a run's columns of the tile
-  float* part_ssq;       // [slot][T] .. and of x_next^2
+  float* part;           // [row][M] sums of x_next . phi^T over a run's columns of the tile
+  float* part_ssq;       // [row] .. and of x_next^2
   int64_t w;             // stages of a block's run
   int rounds;            // whole tiles of every block before its run
   int64_t T;
@@ -430,7 +427,9 @@ __global__ __launch_bounds__(kPPThreads) void post_pre_fwd_kernel(PostPreArgs a)
             }
             if (q == 0) inv_sh[16 * rb + r] = inv_row;
           } else {
-            const int64_t at = (cc.tile < left0 ? 0 : (int64_t)blockIdx.x - (cc.tile - left0) * nst / a.w) * T + tb + 16 * rb;
+            // row of the sums: a token of a whole tile has one, those after have `slots` (post_pre_plan)
+            const int64_t slot = cc.tile < left0 ? 0 : (int64_t)blockIdx.x - (cc.tile - left0) * nst / a.w;
+            const int64_t at = slot * (T - left0 * TT) + tb + 16 * rb;
 #pragma unroll
             for (int v = 0; v < 4; ++v)
 #pragma unroll
@@ -495,40 +494,10 @@ bool post_pre_usable(const void* x, const void* h_out, const void* phi, const vo
 
 using namespace mhc;
 
-namespace {
-// One block a CU (its LDS).  Whole tiles in rounds over all CUs, in an order
-// that keeps the blocks on neighbouring tiles (runs of several tiles a block
-// were 10% slower at D = 2048), then runs of equal length over the tiles left;
-// at most about 64 slots of sums a tile for the finish kernel to add.
-struct PostPrePlan {
-  int64_t w = 1, blocks = 0;
-  int rounds = 0;
-  bool whole_rounds = false;
-  size_t ssq_off = 0, y_off = 0, bytes = 0;
-};
-PostPrePlan post_pre_plan(int64_t T, int32_t D) {
-  PostPrePlan p;
-  if (T <= 0) return p;
-  const int64_t nst = D / kPPCW, ntiles = (T + kPPTile - 1) / kPPTile, cus = device_cu_count();
-  p.rounds = (int)(ntiles / cus);
-  const int64_t total = (ntiles - p.rounds * cus) * nst;
-  p.w = (total + cus - 1) / cus;
-  if (p.w < (nst + 63) / 64) p.w = (nst + 63) / 64;
-  p.blocks = p.rounds ? cus : (total + p.w - 1) / p.w;
-  p.whole_rounds = total == 0;
-  int64_t slots = total ? (nst + p.w - 1) / p.w + 1 : 1;
-  if (slots > p.blocks) slots = p.blocks;
-  p.ssq_off = align256((size_t)slots * T * kPPM * 4);
-  p.y_off = p.ssq_off + align256((size_t)slots * T * 4);
-  p.bytes = p.y_off + fwd_y_ws_bytes(T, kPPN);
-  return p;
-}
-}  // namespace
-
 extern "C" size_t mhc_post_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, int32_t phi_dtype) {
   const size_t pre = mhc_pre_fwd_workspace_size(T, N, D, phi_dtype);
   if (N != kPPN || phi_dtype != MHC_DTYPE_BF16 || D < kPPMinD || D % kPPCW || T <= 0) return pre;
-  const size_t own = post_pre_plan(T, D).bytes;
+  const size_t own = post_pre_plan(T, D, device_cu_count()).bytes;
   return own > pre ? own : pre;
 }
 
@@ -558,7 +527,7 @@ extern "C" int mhc_post_pre_fwd_ex(const void* x, const float* h_res, const void
     if (rc || used) return rc;
   }
   const bool usable = post_pre_usable(x, h_out, phi, x_next, y, x_dtype, phi_dtype, N, D);
-  const PostPrePlan p = usable ? post_pre_plan(T, D) : PostPrePlan{};
+  const PostPrePlan p = usable ? post_pre_plan(T, D, device_cu_count()) : PostPrePlan{};
   if (!usable || !workspace || workspace_bytes < p.bytes ||
       pre_fwd_single_pass_applies(x_next, x_dtype, phi, phi_dtype, y, workspace_bytes, T, N, D,
                                   (hipStream_t)stream)) {

@@ -69,7 +69,7 @@ struct PreFwdArgs {
   const void* phi_raw;
   int gen_nst, gen_tt;
   int64_t gen_w;
-  int64_t gen_whole;  // tiles before the runs, summed by one block each
+  int64_t gen_whole;  // tiles before the runs, summed by one block each: their tokens have one slot
   // single-pass form: its status word (nonzero when a bounded wait timed
   // out); the finalize kernel then writes NaN to every output of the call
   // and copies the word to status_out (the caller's, may be null)
@@ -872,6 +872,9 @@ __device__ __forceinline__ int fwd_slots(const PreFwdArgs& a, int64_t tok, int n
   if (tile < 0) return 1;
   return (int)(((tile + 1) * a.gen_nst - 1) / a.gen_w - tile * a.gen_nst / a.gen_w) + 1;
 }
+// Rows of sums between a token's slots (row t in slot 0): those of the tokens
+// that have several.
+__device__ __forceinline__ int64_t fwd_slot_rows(const PreFwdArgs& a) { return a.T - a.gen_whole * a.gen_tt; }
 
 // ---- split-K form, kernels 2 and 3 -----------------------------------------
 // Kernel 2: one N x N lane group per token sums the splits' partials in split
@@ -891,9 +894,10 @@ __global__ __launch_bounds__(kFwdThreads) void pre_fwd_finalize_kernel(PreFwdArg
   // unrolled iterations issue together instead of waiting one by one
   const int eh = e < 2 * N ? e : 0;
   const int ns = fwd_slots(a, tk, nsplit);
+  const int64_t slot_rows = fwd_slot_rows(a);
 #pragma unroll 8
   for (int s = 0; s < ns; ++s) {
-    const int64_t row = (int64_t)s * T + tk;
+    const int64_t row = s * slot_rows + tk;
     ssq += a.part_ssq[row];
     acc_l += a.part[row * M + 2 * N + e];
     acc_h += a.part[row * M + eh];

@@ -416,14 +416,14 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_finish_kernel(Pr
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int groups = blockDim.x / VP, yw = blockDim.x / kWave - 1;
-  const int64_t t = blockIdx.x, T = a.T;
+  const int64_t t = blockIdx.x;
   const int ns = fwd_slots(a, t, nsplit);
   {
     const int v = tid % VP, g = tid / VP;
     float sum = 0.f;
     if (v <= M) {
       const float* p = v < M ? a.part + t * M + v : a.part_ssq + t;
-      const int64_t stride = v < M ? T * M : T;
+      const int64_t rows = fwd_slot_rows(a), stride = v < M ? rows * M : rows;
 #pragma unroll 4
       for (int s = g; s < ns; s += groups) sum += p[s * stride];
     }

@@ -1,5 +1,5 @@
 // Work split and workspace layout of the pre forward's general contraction
-// (pre_fwd_gen.hpp).  Plain host C++ with no HIP in it: a test compiles it
+// (pre_fwd_gen.hpp) and of the fused post + pre forward (post_pre.hip).  Plain host C++ with no HIP in it: a test compiles it
 // alone and walks the layouts of many shapes on the CPU.
 #pragma once
 
@@ -75,5 +75,44 @@ inline int64_t gen_chunk(int64_t T, int N, int D, int cus, size_t bytes) {
 
 // Workspace of the general form for all T tokens at once.
 inline size_t gen_ws_bytes(int64_t T, int N, int D, int cus) { return kPreFwdWsBase + gen_plan(T, N, D, cus).bytes; }
+
+// ---- fused post + pre forward ------------------------------------------------
+constexpr int kPPN = 4, kPPM = 24;  // streams, and columns of mixes
+constexpr int kPPTile = 32;         // tokens of a tile
+constexpr int kPPCW = 64;           // columns of a stage
+
+// One block a CU (its LDS).  Whole tiles in rounds over all CUs, in an order
+// that keeps the blocks on neighbouring tiles (runs of several tiles a block
+// were 10% slower at D = 2048), then runs of equal length over the tiles left;
+// at most about 64 slots of sums a tile for the finish kernel to add.  A token
+// t of the whole tiles has one row of sums, row t; the `left` after them have
+// `slots`, row s * left + t in slot s.
+struct PostPrePlan {
+  int64_t w = 1, blocks = 0, left = 0;
+  int rounds = 0, slots = 1;
+  bool whole_rounds = false;
+  size_t ssq_off = 0, y_off = 0, bytes = 0;
+};
+inline PostPrePlan post_pre_plan(int64_t T, int32_t D, int cus) {
+  PostPrePlan p;
+  if (T <= 0) return p;
+  const int64_t nst = D / kPPCW, ntiles = (T + kPPTile - 1) / kPPTile;
+  p.rounds = (int)(ntiles / cus);
+  const int64_t whole = (int64_t)p.rounds * cus, total = (ntiles - whole) * nst;
+  p.w = (total + cus - 1) / cus;
+  if (p.w < (nst + 63) / 64) p.w = (nst + 63) / 64;
+  p.blocks = p.rounds ? cus : (total + p.w - 1) / p.w;
+  p.whole_rounds = total == 0;
+  if (total) {
+    p.left = T - whole * kPPTile;
+    p.slots = (int)((nst + p.w - 1) / p.w) + 1;
+    if (p.slots > p.blocks) p.slots = (int)p.blocks;
+  }
+  const int64_t rows = T - p.left + p.slots * p.left;
+  p.ssq_off = align256((size_t)rows * kPPM * 4);
+  p.y_off = p.ssq_off + align256((size_t)rows * 4);
+  p.bytes = p.y_off + fwd_y_ws_bytes(T, kPPN);
+  return p;
+}
 
 }  // namespace mhc

@@ -39,10 +39,11 @@ int launch_pre_y_pass(const void* x, const float* pre, void* y, int64_t T, int N
 // 16-byte aligned rows: a token's sums in slots (runs of `w` stages, `nst`
 // stages a tile of `tt` tokens: the blocks whose runs touch the token's tile),
 // then heads, Sinkhorn and y.  `ws`: fwd_y_ws_bytes of scratch.  The fused
-// post + pre forward runs it on x_next.  The first `whole` tiles have one slot.
+// post + pre forward runs it on x_next.  The first `whole` tiles have one
+// slot; slot s of a token t after them is row s * (T - whole * tt) + t.
 struct PreFinish {
   const void* x;
-  float *part, *part_ssq;  // [slot][T][24], [slot][T]
+  float *part, *part_ssq;  // [row][24], [row]
   char* ws;
   int nst, tt;
   int64_t w, whole;

@@ -64,3 +64,36 @@ def test_less_workspace_runs_the_two_operators():
     assert torch.equal(x_next, xw)
     _close(post, want["post_out"], "post_out")
     _close(comb, want["comb_frag"], "comb_frag")
+
+
+def _c_call(x, h_res, h_out, h_post, phi, alpha, base, ws, size):
+    """mhc_post_pre_fwd in the first `size` bytes of ws: (x_next, dict)."""
+    T, N, D = x.shape
+    f32 = dict(device=DEV, dtype=torch.float32)
+    x_next, y = torch.empty_like(x), torch.empty(T, D, device=DEV, dtype=BF)
+    o = {"post_out": torch.empty(T, N, **f32), "comb_frag": torch.empty(T, N, N, **f32), "inv_rms": torch.empty(T, **f32),
+         "mixes": torch.empty(T, 24, **f32), "h_res_logits": torch.empty(T, N, N, **f32), "pre": torch.empty(T, N, **f32)}
+    rc = _lib.load().mhc_post_pre_fwd(
+        x.data_ptr(), h_res.data_ptr(), h_out.data_ptr(), h_post.data_ptr(), 1, phi.data_ptr(), 1, alpha.data_ptr(),
+        base.data_ptr(), 1e-6, 1e-6, -10.0, 10.0, 20, x_next.data_ptr(), y.data_ptr(), *(t.data_ptr() for t in o.values()),
+        ws.data_ptr(), size, T, N, D, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "mhc_post_pre_fwd")
+    return x_next, dict(o, y=y)
+
+
+@pytest.mark.parametrize("T,D", [(1, 256), (100, 7168), (3000, 1024), (8193, 256), (8225, 448), (16500, 512), (24700, 5120)])
+def test_sums_stay_in_the_workspace(T, D):
+    """The workspace that is asked for, with a guard region behind it."""
+    print(f"[post_pre runs] guarded workspace T={T} D={D}", flush=True)
+    x, h_res, h_out, h_post, _ = post_inputs(T, 4, D, BF, seed=T)
+    _, phi, alpha, base, *_ = pre_inputs(1, 4, D, BF, BF, seed=D)
+    size, guard = _lib.load().mhc_post_pre_fwd_workspace_size(T, 4, D, 1), 4 << 20
+    ws = torch.full((size + guard,), 0x5a, dtype=torch.uint8, device=DEV)
+    x_next, out = _c_call(x, h_res, h_out, h_post, phi, alpha, base, ws, size)
+    y = m.mhc_post(x, h_res, h_out, h_post)
+    want = m.mhc_pre_clamp_sinkhorn(y, phi, alpha, base, need_backward=True, **KW)
+    torch.cuda.synchronize()
+    assert bool((ws[size:] == 0x5a).all())
+    assert torch.equal(x_next, y)
+    for k in FWD_KEYS:
+        _close(out[k], want[k], f"T={T} D={D} {k}")

@@ -1,8 +1,9 @@
-"""The general pre forward's plan (csrc/pre_fwd_plan.hpp), on the CPU: whatever
-workspace a caller gives, every sum that a block of any chunk writes, and the
-chunk's pre and inv_rms, lie inside it, in regions of their own.  The walk
-repeats the kernel's indexing: block b takes stages b * w .. of the tiles, and
-its sums of a tile go to slot b - tile * nst / w."""
+"""The plans of the general pre forward and of the fused post + pre forward
+(csrc/pre_fwd_plan.hpp), on the CPU: whatever workspace a caller gives, every
+sum that a block of any chunk writes, and the chunk's pre and inv_rms, lie
+inside it, in regions of their own.  The walks repeat the kernels' indexing:
+block b takes stages b * w .. of the tiles (fused: of those left after whole
+rounds), and its sums of a tile go to slot b - tile * nst / w."""
 
 from __future__ import annotations
 
@@ -13,6 +14,7 @@ import subprocess
 import pytest
 
 from conftest import PKG_DIR
+from FlagOS_mhc import _lib
 
 WALK = r"""
 #include <stdio.h>
@@ -57,12 +59,39 @@ static void walk(int64_t T, int N, int D, int cus, size_t bytes) {
   }
 }
 
+// the fused forward: no row of sums written twice, none past its region, and
+// no more of them than a few for every token that runs share
+static void walk_fused(int64_t T, int D, int cus) {
+  const PostPrePlan p = post_pre_plan(T, D, cus);
+  const int64_t nst = D / kPPCW, ntiles = (T + kPPTile - 1) / kPPTile, left0 = p.rounds * p.blocks;
+  const int64_t total = (ntiles - left0) * nst, regions = (int64_t)(p.ssq_off / (4 * kPPM));
+  if (p.whole_rounds != (total == 0)) fail("rounds", T, kPPN, D, p.bytes, T);
+  if (p.left != (total ? T - left0 * kPPTile : 0)) fail("left", T, kPPN, D, p.bytes, T);
+  int64_t last = left0 * kPPTile < T ? left0 * kPPTile : T, covered = 0;  // rows of the whole tiles
+  for (int64_t b = 0; b < p.blocks; ++b) {
+    const int64_t u0 = b * p.w, u1 = u0 + p.w < total ? u0 + p.w : total;
+    if (u0 < u1) covered += u1 - u0;
+    for (int64_t i = u0 / nst; u0 < u1 && i <= (u1 - 1) / nst; ++i) {  // tile left0 + i
+      const int64_t slot = b - i * nst / p.w;
+      const int64_t n = (left0 + i + 1) * kPPTile < T ? (left0 + i + 1) * kPPTile : T;
+      if (slot < 0 || slot >= ((i + 1) * nst - 1) / p.w - i * nst / p.w + 1) fail("slot", T, kPPN, D, p.bytes, T);
+      if (slot * p.left + n > last) last = slot * p.left + n;
+    }
+  }
+  if (covered != total) fail("stages without a block", T, kPPN, D, p.bytes, T);
+  if (last > regions || p.ssq_off + last * 4 > p.y_off) fail("sums past their region", T, kPPN, D, p.bytes, T);
+  if (p.y_off + fwd_y_ws_bytes(T, kPPN) > p.bytes) fail("pre past the workspace", T, kPPN, D, p.bytes, T);
+  if ((int64_t)p.bytes > (T + 3 * (int64_t)kPPTile * cus) * 100 + 20 * T + 2048) fail("too much", T, kPPN, D, p.bytes, T);
+}
+
 int main() {
   // last chunks whose own plan would have shorter runs, and so more slots,
   // than a whole chunk's
   walk(16512, 4, 256, 256, 4326656);
   walk(8297, 4, 512, 256, 3900000);
   walk(16157, 4, 1040, 256, 5170944);
+  walk_fused(65537, 5120, 256);
+  walk_fused(131104, 5120, 256);
   std::mt19937_64 rng(1);
   auto uni = [&](double a, double b) { return a + (b - a) * (double)(rng() >> 11) / 9007199254740992.0; };
   auto logu = [&](double a, double b) { return (int64_t)exp2(uni(log2(a), log2(b))); };
@@ -72,6 +101,7 @@ int main() {
     const size_t full = gen_ws_bytes(T, N, D, cus);
     walk(T, N, D, cus, full);
     walk(T, N, D, cus, (size_t)(full * uni(0.02, 1.0)));
+    walk_fused(T, (int)(64 * logu(4, 160)), cus);
     // exactly what some chunk needs
     const int64_t c = gen_chunk(T, N, D, cus, (size_t)(full * uni(0.05, 1.0)));
     if (c > 0) walk(T, N, D, cus, gen_ws_bytes(c, N, D, cus));
@@ -92,3 +122,12 @@ def test_every_chunk_stays_in_the_workspace(tmp_path):
                     str(exe)], check=True)
     p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=100)
     assert p.returncode == 0, p.stdout
+
+
+@pytest.mark.parametrize("T,D", [(65537, 5120), (65568, 2048), (131104, 5120), (8193, 256)])
+def test_fused_workspace_of_a_token_more_than_whole_rounds(T, D):
+    """The slots of the runs are those of the tokens left after whole rounds
+    (at most 8192 tokens and their sums twice over), not of all tokens."""
+    lib = _lib.load()
+    most = lib.mhc_pre_fwd_workspace_size(T, 4, D, 1) + 100 * (T + 3 * 8192) + 20 * T
+    assert lib.mhc_post_pre_fwd_workspace_size(T, 4, D, 1) <= most
