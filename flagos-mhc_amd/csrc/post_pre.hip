@@ -24,7 +24,10 @@
 // next tile's loads.  Measured (bf16, us, whole operator, a tile a block as
 // before / now; MI355X): D = 7168: T = 64 152 / 15, T = 1024 168 / 50, T = 4096
 // 222 / 165, T = 9000 461 / 345, T = 8192 312 / 312; D = 5120, T = 5999 182 /
-// 172.  (A tile's gates sit in one of two LDS buffers; with D >= 64 S a buffer
+// 172.  Without room for the sums the tiles left go whole, one a block, too
+// (post + pre in turn / so: D = 512, T = 500 26.0 / 20.4; D = 5120, T = 1024
+// 139 / 123, T = 4096 207 / 158; slower only just past a round: T = 9000, D =
+// 2048 140 / 166).  (A tile's gates sit in one of two LDS buffers; with D >= 64 S a buffer
 // is free again before the tile after the next one is loaded.)
 //
 // A block (8 waves, two per SIMD so that one wave's waits overlap the other's
@@ -527,7 +530,8 @@ extern "C" int mhc_post_pre_fwd_ex(const void* x, const float* h_res, const void
     if (rc || used) return rc;
   }
   const bool usable = post_pre_usable(x, h_out, phi, x_next, y, x_dtype, phi_dtype, N, D);
-  const PostPrePlan p = usable ? post_pre_plan(T, D, device_cu_count()) : PostPrePlan{};
+  PostPrePlan p = usable ? post_pre_plan(T, D, device_cu_count()) : PostPrePlan{};
+  if (usable && workspace_bytes < p.bytes) p = post_pre_plan(T, D, device_cu_count(), true);
   if (!usable || !workspace || workspace_bytes < p.bytes ||
       pre_fwd_single_pass_applies(x_next, x_dtype, phi, phi_dtype, y, workspace_bytes, T, N, D,
                                   (hipStream_t)stream)) {
@@ -555,8 +559,7 @@ extern "C" int mhc_post_pre_fwd_ex(const void* x, const float* h_res, const void
   a.rounds = p.rounds;
   a.T = T;
   a.D = D;
-  const bool heads = p.whole_rounds;
-  if (heads) {
+  if (p.heads) {
     a.alpha = alpha;
     a.base = base;
     a.norm_eps = norm_eps;

@@ -86,31 +86,33 @@ constexpr int kPPCW = 64;           // columns of a stage
 // were 10% slower at D = 2048), then runs of equal length over the tiles left;
 // at most about 64 slots of sums a tile for the finish kernel to add.  A token
 // t of the whole tiles has one row of sums, row t; the `left` after them have
-// `slots`, row s * left + t in slot s.
+// `slots`, row s * left + t in slot s.  With whole rounds only, or with
+// `whole_tiles` (a tile left a block, for a workspace without room for sums),
+// the kernel runs the heads itself and keeps none.
 struct PostPrePlan {
   int64_t w = 1, blocks = 0, left = 0;
-  int rounds = 0, slots = 1;
-  bool whole_rounds = false;
+  int rounds = 0, slots = 0;
+  bool heads = false;
   size_t ssq_off = 0, y_off = 0, bytes = 0;
 };
-inline PostPrePlan post_pre_plan(int64_t T, int32_t D, int cus) {
+inline PostPrePlan post_pre_plan(int64_t T, int32_t D, int cus, bool whole_tiles = false) {
   PostPrePlan p;
   if (T <= 0) return p;
   const int64_t nst = D / kPPCW, ntiles = (T + kPPTile - 1) / kPPTile;
   p.rounds = (int)(ntiles / cus);
   const int64_t whole = (int64_t)p.rounds * cus, total = (ntiles - whole) * nst;
-  p.w = (total + cus - 1) / cus;
+  p.heads = whole_tiles || total == 0;
+  p.w = p.heads ? nst : (total + cus - 1) / cus;
   if (p.w < (nst + 63) / 64) p.w = (nst + 63) / 64;
   p.blocks = p.rounds ? cus : (total + p.w - 1) / p.w;
-  p.whole_rounds = total == 0;
-  if (total) {
+  if (!p.heads) {
     p.left = T - whole * kPPTile;
     p.slots = (int)((nst + p.w - 1) / p.w) + 1;
     if (p.slots > p.blocks) p.slots = (int)p.blocks;
+    const int64_t rows = T - p.left + p.slots * p.left;
+    p.ssq_off = align256((size_t)rows * kPPM * 4);
+    p.y_off = p.ssq_off + align256((size_t)rows * 4);
   }
-  const int64_t rows = T - p.left + p.slots * p.left;
-  p.ssq_off = align256((size_t)rows * kPPM * 4);
-  p.y_off = p.ssq_off + align256((size_t)rows * 4);
   p.bytes = p.y_off + fwd_y_ws_bytes(T, kPPN);
   return p;
 }

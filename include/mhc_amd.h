@@ -277,8 +277,10 @@ int mhc_pre_bwd_ex(const void* x, int32_t x_dtype, const void* phi, int32_t phi_
  * that kernel forms x_next itself (x and h_out read once, x_next written
  * once; outputs bit-identical to the two operators); other shapes with
  * D % 64 == 0 and D >= 256 read x once and write x_next once, then read
- * x_next back for y; every other shape, and a workspace smaller than
- * mhc_post_pre_fwd_workspace_size, runs mhc_post_fwd then mhc_pre_fwd.
+ * x_next back for y, in whole tiles of 32 tokens only (slower where they do
+ * not fill the GPU) if the workspace is smaller than
+ * mhc_post_pre_fwd_workspace_size but holds 16 and 4 bytes a token, each
+ * rounded up to 256; every other shape runs mhc_post_fwd then mhc_pre_fwd.
  */
 size_t mhc_post_pre_fwd_workspace_size(int64_t T, int32_t N, int32_t D, int32_t phi_dtype);
 int mhc_post_pre_fwd(const void* x, const float* h_res, const void* h_out, const float* h_post,

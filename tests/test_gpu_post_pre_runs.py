@@ -43,7 +43,7 @@ def test_runs_match_the_two_operators(T, D):
     assert bool(((out["y"].float() - want["y"].float()).abs() <= 2e-2 + 2e-2 * want["y"].float().abs()).all())
 
 
-def test_less_workspace_runs_the_two_operators():
+def test_less_workspace_gives_the_same_results():
     T, N, D, M = 500, 4, 512, 24
     x, h_res, h_out, h_post, _ = post_inputs(T, N, D, BF, seed=1)
     _, phi, alpha, base, *_ = pre_inputs(1, N, D, BF, BF, seed=2)
@@ -51,7 +51,7 @@ def test_less_workspace_runs_the_two_operators():
     f32 = dict(device=DEV, dtype=torch.float32)
     x_next, y = torch.empty_like(x), torch.empty(T, D, device=DEV, dtype=BF)
     post, comb = torch.empty(T, N, **f32), torch.empty(T, N, N, **f32)
-    size = 256 + T * 20 + 512  # what the pre forward's two kernels need
+    size = 256 + T * 20 + 512  # pre and inv_rms, no room for sums
     assert size < lib.mhc_post_pre_fwd_workspace_size(T, N, D, 1)
     ws = torch.empty(size, dtype=torch.uint8, device=DEV)
     rc = lib.mhc_post_pre_fwd(x.data_ptr(), h_res.data_ptr(), h_out.data_ptr(), h_post.data_ptr(), 1, phi.data_ptr(), 1,
@@ -97,3 +97,25 @@ def test_sums_stay_in_the_workspace(T, D):
     assert torch.equal(x_next, y)
     for k in FWD_KEYS:
         _close(out[k], want[k], f"T={T} D={D} {k}")
+
+
+@pytest.mark.parametrize("T,D", [(1, 256), (33, 7168), (500, 512), (8193, 256), (9000, 1024), (16500, 320)])
+def test_whole_tiles_without_room_for_sums(T, D):
+    """A workspace that holds pre and inv_rms only: the fused kernel in whole
+    tiles, one a block in the last round (it leaves pre at the workspace's
+    start; the two operators in turn do not)."""
+    print(f"[post_pre runs] whole tiles T={T} D={D}", flush=True)
+    x, h_res, h_out, h_post, _ = post_inputs(T, 4, D, BF, seed=T)
+    _, phi, alpha, base, *_ = pre_inputs(1, 4, D, BF, BF, seed=D)
+    size, guard = (16 * T + 255) // 256 * 256 + (4 * T + 255) // 256 * 256, 1 << 20
+    ws = torch.full((size + guard,), 0x5a, dtype=torch.uint8, device=DEV)
+    x_next, out = _c_call(x, h_res, h_out, h_post, phi, alpha, base, ws, size)
+    y = m.mhc_post(x, h_res, h_out, h_post)
+    want = m.mhc_pre_clamp_sinkhorn(y, phi, alpha, base, need_backward=True, **KW)
+    torch.cuda.synchronize()
+    assert bool((ws[size:] == 0x5a).all())
+    assert torch.equal(ws[:16 * T].view(torch.float32), out["pre"].reshape(-1))
+    assert torch.equal(x_next, y)
+    for k in FWD_KEYS:
+        _close(out[k], want[k], f"T={T} D={D} {k}")
+    assert bool(((out["y"].float() - want["y"].float()).abs() <= 2e-2 + 2e-2 * want["y"].float().abs()).all())

@@ -61,12 +61,12 @@ static void walk(int64_t T, int N, int D, int cus, size_t bytes) {
 
 // the fused forward: no row of sums written twice, none past its region, and
 // no more of them than a few for every token that runs share
-static void walk_fused(int64_t T, int D, int cus) {
-  const PostPrePlan p = post_pre_plan(T, D, cus);
+static void walk_fused(int64_t T, int D, int cus, bool whole_tiles) {
+  const PostPrePlan p = post_pre_plan(T, D, cus, whole_tiles);
   const int64_t nst = D / kPPCW, ntiles = (T + kPPTile - 1) / kPPTile, left0 = p.rounds * p.blocks;
   const int64_t total = (ntiles - left0) * nst, regions = (int64_t)(p.ssq_off / (4 * kPPM));
-  if (p.whole_rounds != (total == 0)) fail("rounds", T, kPPN, D, p.bytes, T);
-  if (p.left != (total ? T - left0 * kPPTile : 0)) fail("left", T, kPPN, D, p.bytes, T);
+  if (p.heads != (whole_tiles || total == 0)) fail("heads", T, kPPN, D, p.bytes, T);
+  if (!p.heads && p.left != T - left0 * kPPTile) fail("left", T, kPPN, D, p.bytes, T);
   int64_t last = left0 * kPPTile < T ? left0 * kPPTile : T, covered = 0;  // rows of the whole tiles
   for (int64_t b = 0; b < p.blocks; ++b) {
     const int64_t u0 = b * p.w, u1 = u0 + p.w < total ? u0 + p.w : total;
@@ -75,12 +75,14 @@ static void walk_fused(int64_t T, int D, int cus) {
       const int64_t slot = b - i * nst / p.w;
       const int64_t n = (left0 + i + 1) * kPPTile < T ? (left0 + i + 1) * kPPTile : T;
       if (slot < 0 || slot >= ((i + 1) * nst - 1) / p.w - i * nst / p.w + 1) fail("slot", T, kPPN, D, p.bytes, T);
+      if (p.heads && (i * nst < u0 || (i + 1) * nst > u1)) fail("part of a tile", T, kPPN, D, p.bytes, T);
       if (slot * p.left + n > last) last = slot * p.left + n;
     }
   }
   if (covered != total) fail("stages without a block", T, kPPN, D, p.bytes, T);
-  if (last > regions || p.ssq_off + last * 4 > p.y_off) fail("sums past their region", T, kPPN, D, p.bytes, T);
+  if (!p.heads && (last > regions || p.ssq_off + last * 4 > p.y_off)) fail("sums past their region", T, kPPN, D, p.bytes, T);
   if (p.y_off + fwd_y_ws_bytes(T, kPPN) > p.bytes) fail("pre past the workspace", T, kPPN, D, p.bytes, T);
+  if (p.heads && p.bytes > fwd_y_ws_bytes(T, kPPN)) fail("more than pre and inv_rms", T, kPPN, D, p.bytes, T);
   if ((int64_t)p.bytes > (T + 3 * (int64_t)kPPTile * cus) * 100 + 20 * T + 2048) fail("too much", T, kPPN, D, p.bytes, T);
 }
 
@@ -90,8 +92,10 @@ int main() {
   walk(16512, 4, 256, 256, 4326656);
   walk(8297, 4, 512, 256, 3900000);
   walk(16157, 4, 1040, 256, 5170944);
-  walk_fused(65537, 5120, 256);
-  walk_fused(131104, 5120, 256);
+  for (int whole = 0; whole < 2; ++whole) {
+    walk_fused(65537, 5120, 256, whole);
+    walk_fused(131104, 5120, 256, whole);
+  }
   std::mt19937_64 rng(1);
   auto uni = [&](double a, double b) { return a + (b - a) * (double)(rng() >> 11) / 9007199254740992.0; };
   auto logu = [&](double a, double b) { return (int64_t)exp2(uni(log2(a), log2(b))); };
@@ -101,7 +105,7 @@ int main() {
     const size_t full = gen_ws_bytes(T, N, D, cus);
     walk(T, N, D, cus, full);
     walk(T, N, D, cus, (size_t)(full * uni(0.02, 1.0)));
-    walk_fused(T, (int)(64 * logu(4, 160)), cus);
+    walk_fused(T, (int)(64 * logu(4, 160)), cus, rng() & 1);
     // exactly what some chunk needs
     const int64_t c = gen_chunk(T, N, D, cus, (size_t)(full * uni(0.05, 1.0)));
     if (c > 0) walk(T, N, D, cus, gen_ws_bytes(c, N, D, cus));
