@@ -60,12 +60,14 @@ inline GenPlan gen_plan(int64_t T, int N, int D, int cus) {
 
 // Tokens a call of the general form takes at a time in `bytes` of workspace:
 // all of them, or a multiple of the tile of at least kGenMinChunk (below that
-// 0: the caller runs the form that needs no sums in memory).
-constexpr int64_t kGenMinChunk = 4096;
+// 0: the caller runs the form that needs no sums in memory).  At most
+// kGenMaxChunk: the kernels after the contraction have a block of up to 1024
+// threads a token, and a dispatch less than 2^32 threads.
+constexpr int64_t kGenMinChunk = 4096, kGenMaxChunk = ((int64_t)1 << 22) - 128;
 inline int64_t gen_chunk(int64_t T, int N, int D, int cus, size_t bytes) {
   if (bytes <= kPreFwdWsBase) return 0;
   bytes -= kPreFwdWsBase;
-  int64_t c = T;
+  int64_t c = T < kGenMaxChunk ? T : kGenMaxChunk;
   while (gen_plan(c, N, D, cus).bytes > bytes) {
     c = round_up(c / 2, 128);
     if (c < kGenMinChunk || c >= T) return 0;
@@ -73,8 +75,10 @@ inline int64_t gen_chunk(int64_t T, int N, int D, int cus, size_t bytes) {
   return c;
 }
 
-// Workspace of the general form for all T tokens at once.
-inline size_t gen_ws_bytes(int64_t T, int N, int D, int cus) { return kPreFwdWsBase + gen_plan(T, N, D, cus).bytes; }
+// Workspace of the general form's largest chunk of T tokens.
+inline size_t gen_ws_bytes(int64_t T, int N, int D, int cus) {
+  return kPreFwdWsBase + gen_plan(T < kGenMaxChunk ? T : kGenMaxChunk, N, D, cus).bytes;
+}
 
 // ---- fused post + pre forward ------------------------------------------------
 constexpr int kPPN = 4, kPPM = 24;  // streams, and columns of mixes

@@ -196,3 +196,16 @@ def test_inv_rms_of_long_runs(T, N, D, dtype):
     got = _pre_forward(x, phi, alpha, base, 1e-6, 1e-6, -10.0, 10.0, 20, True, False)["inv_rms"]
     want = torch.cat([torch.rsqrt(c.double().reshape(len(c), -1).square().mean(1) + 1e-6) for c in x.split(4096)])
     assert float((got.double() - want).norm() / want.norm()) < 3e-7
+
+
+def test_more_tokens_than_a_launch_takes():
+    """A chunk and 777 tokens of a second one, in the workspace that is asked for."""
+    T, N, D = (1 << 22) - 128 + 777, 4, 3
+    print(f"[pre_fwd general] T={T} N={N} D={D}", flush=True)
+    x, phi, alpha, base, *_ = pre_inputs(T, N, D, F32, F32, seed=2)
+    out = _pre_forward(x, phi, alpha, base, 1e-6, 1e-6, -10.0, 10.0, 20, True, True)
+    torch.cuda.synchronize()
+    idx = torch.cat([_subset(T, k=48, seed=T), torch.arange((1 << 22) - 140, (1 << 22) - 110, device=DEV)])
+    want = _oracle_fwd(idx, x, phi, alpha, base, _kw())
+    check_fwd(out, want, F32, idx, "two chunks")
+    assert_close(out["x_scaled"][idx], want["x_scaled"], 1e-5, 1e-6, "x_scaled")

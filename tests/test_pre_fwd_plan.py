@@ -35,6 +35,7 @@ static void walk(int64_t T, int N, int D, int cus, size_t bytes) {
   const int64_t chunk = gen_chunk(T, N, D, cus, bytes);
   if (chunk <= 0) return;
   if (chunk < T) ++chunked;
+  if (chunk * 1024 >= (int64_t)1 << 32) fail("too many threads", T, N, D, bytes, chunk);
   const GenPlan p = gen_plan(chunk, N, D, cus);
   const size_t room = bytes - kPreFwdWsBase, M = 2 * N + N * N;
   for (int64_t t0 = 0; t0 < T; t0 += chunk) {
@@ -92,6 +93,10 @@ int main() {
   walk(16512, 4, 256, 256, 4326656);
   walk(8297, 4, 512, 256, 3900000);
   walk(16157, 4, 1040, 256, 5170944);
+  // rows of a few elements: more tokens than a dispatch has blocks of 1024 threads for
+  walk(70000000, 4, 8, 256, gen_ws_bytes(70000000, 4, 8, 256));
+  walk(70000000, 8, 3, 256, gen_ws_bytes(70000000, 8, 3, 256) / 3);
+  walk((int64_t)2147483647, 4, 1, 256, gen_ws_bytes(2147483647, 4, 1, 256));
   for (int whole = 0; whole < 2; ++whole) {
     walk_fused(65537, 5120, 256, whole);
     walk_fused(131104, 5120, 256, whole);
