@@ -145,13 +145,12 @@ def workspace(name: str, dev: torch.device, *args):
     return torch.empty((max(n, 1),), dtype=torch.uint8, device=dev), n
 
 
-def pre_fwd_size_code(phi_code: int, phi: torch.Tensor, x: torch.Tensor) -> int:
+def pre_fwd_size_code(x_code: int, phi_code: int, addresses: int) -> int:
     """The phi dtype code to ask mhc_pre_fwd_workspace_size with: bf16 x and phi
-    at 16-byte aligned addresses have kernels of their own, any other pair runs
-    the general form, whose workspace is that of an fp32 phi."""
-    if x.dtype == torch.bfloat16 and not (x.data_ptr() | phi.data_ptr()) & 15:
-        return phi_code
-    return DTYPE_CODE[torch.float32]
+    at 16-byte aligned addresses (or-ed together here) have kernels of their
+    own, any other pair runs the general form, whose workspace is that of an
+    fp32 phi (code 0)."""
+    return phi_code if x_code == 1 and not addresses & 15 else 0
 
 
 def require_device(what: str, *tensors) -> None:

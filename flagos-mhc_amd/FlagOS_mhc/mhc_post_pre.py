@@ -76,8 +76,9 @@ def mhc_post_pre_clamp_sinkhorn(
         pre = torch.empty((T, N), **f32)
     if T > 0:
         lib = _lib.load()
+        xp, pp = x_next.data_ptr(), phi_c.data_ptr()  # the pre forward's operands
         ws, ws_bytes = _lib.workspace("mhc_post_pre_fwd_workspace_size", dev, T, N, D,
-                                      _lib.pre_fwd_size_code(pcode, phi_c, x_next))
+                                      _lib.pre_fwd_size_code(xcode, pcode, xp | pp))
         # the shapes a single pass can take report its bounded waits into a
         # status word, as the pre forward's
         slot = status = None
@@ -87,9 +88,9 @@ def mhc_post_pre_clamp_sinkhorn(
         with _lib.on_device(dev):
             rc = lib.mhc_post_pre_fwd_ex(
                 xf.data_ptr(), hres.data_ptr(), hout.data_ptr(), hpost.data_ptr(), xcode,
-                phi_c.data_ptr(), pcode, alpha_c.data_ptr(), base_c.data_ptr(), float(norm_eps),
+                pp, pcode, alpha_c.data_ptr(), base_c.data_ptr(), float(norm_eps),
                 float(hc_eps), float(clamp_min), float(clamp_max), int(iter_times),
-                x_next.data_ptr(), y.data_ptr(), post_out.data_ptr(), comb.data_ptr(),
+                xp, y.data_ptr(), post_out.data_ptr(), comb.data_ptr(),
                 _lib.ptr(inv_rms), _lib.ptr(mixes), _lib.ptr(logits), _lib.ptr(pre),
                 ws.data_ptr(), ws_bytes, status, T, N, D, _lib.stream_of(xf))
         _lib.check(rc, "mhc_post_pre_clamp_sinkhorn")

@@ -80,8 +80,9 @@ def _pre_forward(x, phi, alpha, base, norm_eps, hc_eps, clamp_min, clamp_max, it
             x_scaled = torch.empty((T, N * D), **f32)
     if T > 0:
         lib = _lib.load()
+        xp, pp = xf.data_ptr(), phi_c.data_ptr()
         ws, ws_bytes = _lib.workspace("mhc_pre_fwd_workspace_size", dev, T, N, D,
-                                      _lib.pre_fwd_size_code(pcode, phi_c, xf))
+                                      _lib.pre_fwd_size_code(xcode, pcode, xp | pp))
         # the shapes the single-pass form can take (N = 4, bf16, T >= 8192;
         # never under stream capture) report its bounded waits into a status word
         slot = status = None
@@ -91,7 +92,7 @@ def _pre_forward(x, phi, alpha, base, norm_eps, hc_eps, clamp_min, clamp_max, it
         stream = _lib.stream_of(xf)
         with _lib.on_device(dev):
             rc = lib.mhc_pre_fwd_ex(
-                xf.data_ptr(), xcode, phi_c.data_ptr(), pcode, alpha_c.data_ptr(),
+                xp, xcode, pp, pcode, alpha_c.data_ptr(),
                 base_c.data_ptr(), float(norm_eps), float(hc_eps), float(clamp_min),
                 float(clamp_max), int(iter_times), y.data_ptr(), post_out.data_ptr(),
                 comb.data_ptr(), _lib.ptr(inv_rms), _lib.ptr(mixes), _lib.ptr(logits),

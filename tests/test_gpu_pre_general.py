@@ -168,7 +168,8 @@ def test_unaligned_bf16_calls_get_the_general_workspace(T, D, which):
         return buf[1:].view(t.shape)
 
     xs, ps = (shifted(x) if which != "phi" else x), (shifted(phi) if which != "x" else phi)
-    assert _lib.pre_fwd_size_code(1, ps, xs) == 0 and _lib.pre_fwd_size_code(1, phi, x) == 1
+    assert _lib.pre_fwd_size_code(1, 1, xs.data_ptr() | ps.data_ptr()) == 0
+    assert _lib.pre_fwd_size_code(1, 1, x.data_ptr() | phi.data_ptr()) == 1
     out = m.mhc_pre_clamp_sinkhorn(xs, ps, alpha, base, **_kw())
     h_res, h_post = want["comb_frag"], want["post_out"]
     h_out = x[:, 0].contiguous()
