@@ -12,7 +12,8 @@
 //   pre_bwd_gpre_kernel, a block per (token, 2048 columns); N = 4 in other
 //   dtypes at T >= 16384: a wave per token here)
 //   Sinkhorn / softmax / clamp / sigmoid-head VJP, lane per matrix element
-//   -> grad_mixes (T,M) and scale[t] = -inv^2 * <grad_mixes, mixes> / (N*D)
+//   -> grad_mixes (T,M) as bf16 planes and, in the (T, N) coefficients beside
+//   pre and inv, scale[t] = -inv^2 * <grad_mixes, mixes> / (N*D)
 //   (because <x, grad_mixes @ phi> = <grad_mixes, mixes> / inv), plus a
 //   per-block partial of grad_alpha / grad_base (fixed summation order).
 // Kernel B, a block per (columns, token split): gs = grad_mixes @ phi on MFMA,
@@ -53,7 +54,6 @@ struct PreBwdSmallArgs {
   int iters;
   const float* pre;
   float* gm;       // (T, M) fp32, or null
-  float* scale;    // (T,), or null
   uint16_t* gmP;   // [2][T][MP32] bf16 planes of grad_mixes, or null
   int64_t gmP_plane;
   uint16_t* gTw;   // [ceil(T/16)][MT][64][2][4] bf16 planes of grad_mixes * inv
@@ -412,7 +412,6 @@ __global__ __launch_bounds__(kBwdThreads) void pre_bwd_small_kernel(PreBwdSmallA
       if (ok && e == 0) *reinterpret_cast<float4*>(a.coefX + tok * 16 + 12) = float4{inv, scale, 0.f, 0.f};
     }
     if (e == 0) {
-      if (ok && a.scale) a.scale[tok] = scale;
       contrib[tt][0] = c0;
       contrib[tt][1] = c1;
       contrib[tt][2] = c2;
@@ -1303,7 +1302,7 @@ __global__ void zero_kernel(float* p, int64_t n) {
 struct BwdLayout {
   int M, L, C, P, MP, MP32, gpre_chunks;
   int64_t K, nblkA, ntiles;
-  size_t off_phiT, off_gm, off_scale, off_partial, off_gphi, off_sink, off_gpre, off_gpl;
+  size_t off_phiT, off_gm, off_partial, off_gphi, off_sink, off_gpre, off_gpl;
   size_t off_gmP, off_gTw, off_coef, total;
   // single-pass form (0 when it cannot apply): G members per group, control
   // words + exchange ring, contribution rows after kernel A's
@@ -1342,7 +1341,8 @@ static int64_t dma_max_splits(int D) {
   return s > kMaxSplits ? s : kMaxSplits;
 }
 
-// Workspace layout.  It covers both forms of kernel B, so the size depends only on (T, N, D, phi dtype, iterations).
+// Workspace layout.  It covers both forms of kernel B, so the size depends only
+// on (T, N, D, phi dtype, iterations).
 static BwdLayout bwd_layout(int64_t T, int N, int D, int32_t phi_dtype, int iters) {
   BwdLayout b{};
   b.M = 2 * N + N * N;
@@ -1357,10 +1357,8 @@ static BwdLayout bwd_layout(int64_t T, int N, int D, int32_t phi_dtype, int iter
   size_t off = 0;
   b.off_phiT = off;
   off += align256(phiT_planes_bytes(phi_dtype, b.M, b.K));
-  b.off_gm = off;
+  b.off_gm = off;  // fp32 grad_mixes: the compensated and the single-pass forms
   off += align256((size_t)T * b.M * 4);
-  b.off_scale = off;
-  off += align256((size_t)T * 4);
   b.bcG = 0;
   if (bc_shape(T, N, D, phi_dtype, &b.bcG)) {
     b.bcMaxg = coop_max_groups(b.bcG);
@@ -1560,7 +1558,6 @@ static int launch_pre_bwd_coop(const BwdLayout& lay, PreBwdSmallArgs sa, const P
   sa.gmP = nullptr;
   sa.gTw = nullptr;
   sa.coef = nullptr;
-  sa.scale = nullptr;
   sa.gpre_part = nullptr;
   sa.coefX = reinterpret_cast<float*>(ws + lay.off_coef);
   hipLaunchKernelGGL((pre_bwd_small_kernel<4, bf16_t, true>), dim3((unsigned)lay.nblkA), dim3(kBwdThreads), 0,
@@ -1614,7 +1611,6 @@ static int launch_pre_bwd(const BwdLayout& lay, PreBwdSmallArgs sa, const PreBwd
     }
   }
   if (!sa.comp) sa.gm = nullptr;  // only the compensated grad_phi reads fp32 grad_mixes
-  sa.scale = nullptr;
   int rc;
   const bool gpre_dma = streaming && sa.T >= kGpreDmaMinT, gpre_split = !gpre_dma && sa.gpre_part;
   if (!phi_ready && !gpre_split && (rc = prepare_phiT_planes(pt, st))) return rc;
@@ -1725,7 +1721,6 @@ static int pre_bwd_entry(const void* x, int32_t x_dtype, const void* phi, int32_
   sa.iters = iter_times;
   sa.pre = pre;
   sa.gm = reinterpret_cast<float*>(ws + lay.off_gm);
-  sa.scale = reinterpret_cast<float*>(ws + lay.off_scale);
   sa.gmP = reinterpret_cast<uint16_t*>(ws + lay.off_gmP);
   sa.gmP_plane = T * lay.MP32;
   sa.gTw = reinterpret_cast<uint16_t*>(ws + lay.off_gTw);
