@@ -31,6 +31,30 @@ namespace mhc {
 
 constexpr int kPostWavesPerBlock = 4;
 
+// 16-byte pieces of rows of D elements.  VECTOR: rows of whole pieces, 16-byte
+// aligned.  Otherwise the last lane of a row takes its last VEC elements again
+// instead of a piece that ends outside it: it stores the same values twice,
+// and the backward's dot products leave the `dup` elements out that the lane
+// before it has (rows of less than VEC elements go one by one).
+template <typename S, bool VECTOR>
+struct PostRows {
+  int D;
+  __device__ __forceinline__ u32x4 ld(const S* row, int d) const {
+    if constexpr (VECTOR)
+      return ld16nt(row + d);
+    else
+      return D < Store<S>::VEC ? ld16_elems(row, D) : ld16nt_u(row + d);
+  }
+  __device__ __forceinline__ void st(S* row, int d, const u32x4& v) const {
+    if constexpr (VECTOR)
+      st16nt(row + d, v);
+    else if (D < Store<S>::VEC)
+      st16_elems(row, D, v);
+    else
+      st16nt_u(row + d, v);
+  }
+};
+
 // MINW: waves per SIMD the register allocation must allow (2 caps the
 // kernel at 256 VGPRs).
 // SUM: the incoming gradient is gy + gy2 (two tensors of gy's layout, added
@@ -60,25 +84,7 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
 
   const int64_t xrow = t * (int64_t)N * D;
   const int64_t hrow = t * (int64_t)D;
-  // VECTOR: rows of whole 16-byte pieces, 16-byte aligned.  Otherwise the last
-  // lane of a row takes its last V elements again instead of a piece that ends
-  // outside it: it stores the same values twice, and the dot products leave
-  // the `dup` elements out that the lane before it has (rows of less than V
-  // elements go one by one).
-  auto ld = [D](const S* row, int d) {
-    if constexpr (VECTOR)
-      return ld16nt(row + d);
-    else
-      return D < Store<S>::VEC ? ld16_elems(row, D) : ld16nt_u(row + d);
-  };
-  auto st = [D](S* row, int d, const u32x4& v) {
-    if constexpr (VECTOR)
-      st16nt(row + d, v);
-    else if (D < Store<S>::VEC)
-      st16_elems(row, D, v);
-    else
-      st16nt_u(row + d, v);
-  };
+  const PostRows<S, VECTOR> rows{D};
 
   if constexpr (VECTOR && N == 8 && std::is_same<S, bf16_t>::value && !SUM) {
     // N = 8: the N*N + N dot products take v_dot2_f32_bf16 on the packed
@@ -136,19 +142,19 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
       const int d = VECTOR || d0 + V <= D || D < V ? d0 : D - V, dup = d0 - d;
       float gv[N][V], xv[N][V], hv[V];
 #pragma unroll
-      for (int i = 0; i < N; ++i) Store<S>::unpack(ld(gy + xrow + (int64_t)i * D, d), gv[i]);
+      for (int i = 0; i < N; ++i) Store<S>::unpack(rows.ld(gy + xrow + (int64_t)i * D, d), gv[i]);
       if constexpr (SUM) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
           float g2[V];
-          Store<S>::unpack(ld(gy2 + xrow + (int64_t)i * D, d), g2);
+          Store<S>::unpack(rows.ld(gy2 + xrow + (int64_t)i * D, d), g2);
 #pragma unroll
           for (int e = 0; e < V; ++e) gv[i][e] += g2[e];
         }
       }
 #pragma unroll
-      for (int j = 0; j < N; ++j) Store<S>::unpack(ld(x + xrow + (int64_t)j * D, d), xv[j]);
-      Store<S>::unpack(ld(h_out + hrow, d), hv);
+      for (int j = 0; j < N; ++j) Store<S>::unpack(rows.ld(x + xrow + (int64_t)j * D, d), xv[j]);
+      Store<S>::unpack(rows.ld(h_out + hrow, d), hv);
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         float o[V];
@@ -159,7 +165,7 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
           for (int i = 0; i < N; ++i) a = fmaf(hr[j * N + i], gv[i][e], a);
           o[e] = a;
         }
-        st(gx + xrow + (int64_t)j * D, d, Store<S>::pack(o));
+        rows.st(gx + xrow + (int64_t)j * D, d, Store<S>::pack(o));
       }
       float oh[V];
 #pragma unroll
@@ -169,7 +175,7 @@ __global__ __launch_bounds__(256, MINW) void post_bwd_kernel(
         for (int i = 0; i < N; ++i) a = fmaf(hp[i], gv[i][e], a);
         oh[e] = a;
       }
-      st(g_hout + hrow, d, Store<S>::pack(oh));
+      rows.st(g_hout + hrow, d, Store<S>::pack(oh));
       if constexpr (!VECTOR) {
 #pragma unroll
         for (int e = 0; e < V; ++e) {
@@ -256,32 +262,14 @@ __global__ __launch_bounds__(kWave * kPostFwdBlockWaves) void post_fwd_block_ker
 #pragma unroll
   for (int i = 0; i < N; ++i) hp[i] = h_post[t * N + i];
   const int64_t xrow = t * (int64_t)N * D, hrow = t * (int64_t)D;
-  // VECTOR: rows of whole 16-byte pieces, 16-byte aligned.  Otherwise the last
-  // lane of a row takes its last V elements again instead of a piece that ends
-  // outside it: it stores the same values twice, and the dot products leave
-  // the `dup` elements out that the lane before it has (rows of less than V
-  // elements go one by one).
-  auto ld = [D](const S* row, int d) {
-    if constexpr (VECTOR)
-      return ld16nt(row + d);
-    else
-      return D < Store<S>::VEC ? ld16_elems(row, D) : ld16nt_u(row + d);
-  };
-  auto st = [D](S* row, int d, const u32x4& v) {
-    if constexpr (VECTOR)
-      st16nt(row + d, v);
-    else if (D < Store<S>::VEC)
-      st16_elems(row, D, v);
-    else
-      st16nt_u(row + d, v);
-  };
+  const PostRows<S, VECTOR> rows{D};
   for (int d0 = wave * CW + lane * V; d0 < D; d0 += W * CW) {
     const int d = VECTOR || d0 + V <= D || D < V ? d0 : D - V;
     float xv[N][V], hv[V];
     if constexpr (V > 1) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) Store<S>::unpack(ld(x + xrow + (int64_t)j * D, d), xv[j]);
-      Store<S>::unpack(ld(h_out + hrow, d), hv);
+      for (int j = 0; j < N; ++j) Store<S>::unpack(rows.ld(x + xrow + (int64_t)j * D, d), xv[j]);
+      Store<S>::unpack(rows.ld(h_out + hrow, d), hv);
     } else {
 #pragma unroll
       for (int j = 0; j < N; ++j) xv[j][0] = load_elem(x, xrow + (int64_t)j * D + d);
@@ -298,7 +286,7 @@ __global__ __launch_bounds__(kWave * kPostFwdBlockWaves) void post_fwd_block_ker
         o[e] = acc;
       }
       if constexpr (V > 1)
-        st(y + xrow + (int64_t)i * D, d, Store<S>::pack(o));
+        rows.st(y + xrow + (int64_t)i * D, d, Store<S>::pack(o));
       else
         store_elem(y, xrow + (int64_t)i * D + d, o[0]);
     }
@@ -329,42 +317,24 @@ __global__ __launch_bounds__(kWave * kPostBlockWaves, MINW) void post_bwd_block_
 #pragma unroll
   for (int i = 0; i < N; ++i) acc_p[i] = 0.f;
   const int64_t xrow = t * (int64_t)N * D, hrow = t * (int64_t)D;
-  // VECTOR: rows of whole 16-byte pieces, 16-byte aligned.  Otherwise the last
-  // lane of a row takes its last V elements again instead of a piece that ends
-  // outside it: it stores the same values twice, and the dot products leave
-  // the `dup` elements out that the lane before it has (rows of less than V
-  // elements go one by one).
-  auto ld = [D](const S* row, int d) {
-    if constexpr (VECTOR)
-      return ld16nt(row + d);
-    else
-      return D < Store<S>::VEC ? ld16_elems(row, D) : ld16nt_u(row + d);
-  };
-  auto st = [D](S* row, int d, const u32x4& v) {
-    if constexpr (VECTOR)
-      st16nt(row + d, v);
-    else if (D < Store<S>::VEC)
-      st16_elems(row, D, v);
-    else
-      st16nt_u(row + d, v);
-  };
+  const PostRows<S, VECTOR> rows{D};
   for (int d0 = wave * CW + lane * V; d0 < D; d0 += W * CW) {
     const int d = VECTOR || d0 + V <= D || D < V ? d0 : D - V, dup = d0 - d;
     float gv[N][V], xv[N][V], hv[V];
 #pragma unroll
-    for (int i = 0; i < N; ++i) Store<S>::unpack(ld(gy + xrow + (int64_t)i * D, d), gv[i]);
+    for (int i = 0; i < N; ++i) Store<S>::unpack(rows.ld(gy + xrow + (int64_t)i * D, d), gv[i]);
     if constexpr (SUM) {
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         float g2[V];
-        Store<S>::unpack(ld(gy2 + xrow + (int64_t)i * D, d), g2);
+        Store<S>::unpack(rows.ld(gy2 + xrow + (int64_t)i * D, d), g2);
 #pragma unroll
         for (int e = 0; e < V; ++e) gv[i][e] += g2[e];
       }
     }
 #pragma unroll
-    for (int j = 0; j < N; ++j) Store<S>::unpack(ld(x + xrow + (int64_t)j * D, d), xv[j]);
-    Store<S>::unpack(ld(h_out + hrow, d), hv);
+    for (int j = 0; j < N; ++j) Store<S>::unpack(rows.ld(x + xrow + (int64_t)j * D, d), xv[j]);
+    Store<S>::unpack(rows.ld(h_out + hrow, d), hv);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       float o[V];
@@ -375,7 +345,7 @@ __global__ __launch_bounds__(kWave * kPostBlockWaves, MINW) void post_bwd_block_
         for (int i = 0; i < N; ++i) a = fmaf(hr[j * N + i], gv[i][e], a);
         o[e] = a;
       }
-      st(gx + xrow + (int64_t)j * D, d, Store<S>::pack(o));
+      rows.st(gx + xrow + (int64_t)j * D, d, Store<S>::pack(o));
     }
     float oh[V];
 #pragma unroll
@@ -385,7 +355,7 @@ __global__ __launch_bounds__(kWave * kPostBlockWaves, MINW) void post_bwd_block_
       for (int i = 0; i < N; ++i) a = fmaf(hp[i], gv[i][e], a);
       oh[e] = a;
     }
-    st(g_hout + hrow, d, Store<S>::pack(oh));
+    rows.st(g_hout + hrow, d, Store<S>::pack(oh));
     if constexpr (!VECTOR) {
 #pragma unroll
       for (int e = 0; e < V; ++e) {
