@@ -500,7 +500,11 @@ __global__ __launch_bounds__(kWave * kFinishWaves) void pre_fwd_gen_y_kernel(Pre
 // 7168 11.6 / 16.2; T = 512 D = 4096 15.0 / 18.0; T = 2048 D = 4096 37.0 / 37.6,
 // D = 256 13.5 / 12.9; T = 16384 D = 256 39 / 26, D = 512 41 / 38, D = 9216 451
 // / 438; fp16 T = 8192 D = 1003 59.6 / 50.5.  N = 8: T = 64 D = 2048 13.6 /
-// 16.1; T = 16384 D = 2048 253 / 262, D = 256 72 / 57.  Four tokens a block
+// 16.1; T = 16384 D = 2048 253 / 262, D = 256 72 / 57.  Narrow rows at few
+// tokens (replayed graphs): N = 4: D = 256, T = 1 8.9 / 10.1, T = 1024 10.0 /
+// 11.3, T = 1536 11.9 / 11.8; D = 512, T = 1024 9.8 / 12.7; fp32 phi, D = 256,
+// T = 1024 10.0 / 12.4; N = 8: D = 256, T = 1 11.4 / 11.8, T = 1024 13.6 / 15.3,
+// T = 1536 15.8 / 15.6; fp32 phi, D = 256, T = 1024 19.0 / 20.7.  Four tokens a block
 // (N = 4, one Sinkhorn wave for the four) gained 0 to 6% above 2048 tokens and
 // lost as much at wide rows.
 static bool finish_applies(int64_t T, int N, int D) { return T <= 1024 || (D >= 512 && (N == 8 || T <= 2048)); }
@@ -520,7 +524,13 @@ static int launch_gen_contraction(const PreFwdArgs& a, const GenPlan& p, hipStre
 template <int N, typename S>
 static int launch_pre_fwd_finish(const PreFwdArgs& a, int nsplit, hipStream_t st) {
   const int chunks = (a.D + 511) / 512;
-  const int yw = chunks < kFinishWaves - 1 ? chunks : kFinishWaves - 1;
+  int yw = chunks < kFinishWaves - 1 ? chunks : kFinishWaves - 1;
+  // N = 8: a group of two waves adds a token's slots (up to 129 of the general
+  // form's), one after the other, and at few tokens the call waits for them:
+  // two groups at least (fp32 phi, D = 1024: T = 1 18.0 -> 14.3 us, T = 256
+  // 26.2 -> 21.3, where finalize + y take 16.6 and 24.6; D = 512, T = 1024 23.4
+  // -> 22.8, but T = 2048 23.9 -> 27.2)
+  if (N == 8 && a.gen_w && a.T <= 1024 && yw < 3) yw = 3;
   const dim3 grid((unsigned)a.T), block(kWave * (1 + yw));
   if (int rc = check_grid(grid, block, "mhc_pre_fwd")) return rc;
   if (a.x_scaled)

@@ -31,6 +31,8 @@ CASES = [
     (2048, 4, 130, HF, F32), (2049, 4, 1003, HF, HF), (8193, 4, 3584, BF, F32), (2049, 8, 517, BF, F32),
     (3000, 8, 1024, F32, F32), (1025, 8, 640, HF, HF), (1030, 8, 333, HF, BF), (1030, 4, 1030, F32, BF),
     (2500, 4, 6001, F32, F32), (66000, 4, 24, BF, F32),
+    # finish blocks of more waves than rows of 512 columns (N = 8, at most 1024 tokens)
+    (1, 8, 1024, BF, F32), (257, 8, 513, F32, F32), (1024, 8, 640, HF, HF),
 ]
 
 
