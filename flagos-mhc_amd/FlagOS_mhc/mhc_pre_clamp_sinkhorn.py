@@ -13,8 +13,9 @@ src/mhc_pre_clamp_sinkhorn.py:974-1022):
    (row, column) normalisations, every denominator being sum + hc_eps
 5. y = sum_n x[:, n, :] * pre[:, n]                        (B,S,D) or (T,D)
 
-``mhc_pre_clamp_sinkhorn`` runs all five stages in one gfx950 kernel
-(``mhc_pre_fwd``): the N*D -> M contraction on bf16 MFMA with fp32
+``mhc_pre_clamp_sinkhorn`` runs the five stages in one call of
+``mhc_pre_fwd_ex``, up to three kernels chosen by size, type and alignment
+(csrc/pre_fwd.hip): the N*D -> M contraction on bf16 MFMA with fp32
 accumulation, the Sinkhorn stage in registers.  It returns the reference's
 dict; with ``need_backward=True`` also inv_rms, x_scaled, mixes,
 h_res_logits (pre-clamp) and pre.

@@ -28,12 +28,14 @@
 // LDS by round-to-nearest adds: one chain over a block's tiles drifts with
 // their number (2-norm error against 64 bits, bf16, one chain / so: N = 8, D =
 // 8191, T = 32768 4.2e-6 / 2.5e-6; N = 4, D = 8191, T = 65536 4.1e-6 / 2.5e-6).
-// No barriers: a wave waits for nothing but its own loads.  It replaces a kernel that staged 32 tokens x 256 columns in LDS (element by
-// element for unaligned rows) between barriers.  Measured, whole backward on
-// MI355X, before -> after: fp16, N = 4, T = 8192: D = 1003 291 -> 115 us, D =
-// 1024 145 -> 80; bf16 T = 16384, D = 907 510 -> 174; fp32 T = 8192, D = 2048
-// 248 -> 215 (this kernel 132: 3.5 TB/s), N = 8, D = 1024 449 -> 271.  Bound
-// by issue at N = 8 (MFMA, conversions) and by loads in flight at N = 4.
+// No barriers: a wave waits for nothing but its own loads.  It replaces a
+// kernel that staged 32 tokens x 256 columns in LDS (element by element for
+// unaligned rows) between barriers.  Measured, whole backward on MI355X, eager,
+// before -> after (in a replayed graph): fp16, N = 4, T = 8192: D = 1003 291 ->
+// 115 us (99), D = 1024 145 -> 80 (66); bf16 T = 16384, D = 907 510 -> 174
+// (145); fp32 T = 8192, D = 2048 248 -> 215 (202; this kernel 132: 3.5 TB/s),
+// N = 8, D = 1024 449 -> 271 (with gs last; 251 in a graph, 246 with gs first).
+// Bound by issue at N = 8 (MFMA, conversions) and by loads in flight at N = 4.
 // What the four rows' loads may not meet is a branch or a use before the next
 // tile's: a wave that joins two streams' columns at load time took twice as
 // long, and the whole grid waits for it.

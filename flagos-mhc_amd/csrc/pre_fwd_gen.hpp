@@ -37,10 +37,10 @@
 //
 // Measured (MI355X, the whole operator; before: one block a 64-token tile
 // that walked all of K with one wave a SIMD, then y): phi fp32, bf16 x, N =
-// 4: D = 7168, T = 1: 177 -> 9.5 us (replayed graph); D = 4096, T = 777: 253
-// -> 24; D = 3584, T = 8193: 250 -> 101 (this kernel 55: 4.2 TB/s of x); fp16
-// x and phi, D = 1003, T = 2049: 312 -> 26; fp32, D = 256, T = 1024: 42 ->
-// 12.  At many tokens issue bounds it as much as memory (splitting phi, the
+// 4: D = 7168, T = 1: 177 -> 9.8 us (now in a replayed graph); D = 4096, T =
+// 777: 253 -> 23; D = 3584, T = 8193: 250 -> 98 (this kernel 55: 4.2 TB/s of
+// x); fp16 x and phi, D = 1003, T = 2049: 312 -> 25; fp32, D = 256, T = 1024:
+// 42 -> 11.  At many tokens issue bounds it as much as memory (splitting phi, the
 // sum of squares, 24 MFMA and 24 LDS reads per wave and stage); two row
 // blocks a wave (half the LDS reads, four waves a block) measured 10% slower,
 // streaming loads 8%, 128-byte row pieces per load instruction 2%.

@@ -1,6 +1,7 @@
 // Work split and workspace layout of the pre forward's general contraction
-// (pre_fwd_gen.hpp) and of the fused post + pre forward (post_pre.hip).  Plain host C++ with no HIP in it: a test compiles it
-// alone and walks the layouts of many shapes on the CPU.
+// (pre_fwd_gen.hpp) and of the fused post + pre forward (post_pre.hip).  Plain
+// host C++ with no HIP in it: a test compiles it alone and walks the layouts of
+// many shapes on the CPU.
 #pragma once
 
 #include <stddef.h>

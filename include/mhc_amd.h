@@ -106,10 +106,11 @@ int mhc_post_bwd_sum_fused(int64_t T, int32_t N, int32_t D, int32_t dtype);
  * x and phi, D = 4096 or 7168 .. 8192 and T >= 8192, the exchange ring of the
  * single-pass form (x read from HBM once, ~13 MB + 120 bytes per token); a
  * smaller workspace that still holds the two-pass forms' runs those.  For phi
- * that is not bf16, or D % 8 != 0, it includes the
- * general form's sums over split columns (at most ~128 * 25 floats a token at
- * few tokens, ~3 * 25 from 16384 on); with less, the tokens run in chunks that
- * fit, or in a slower form that needs only phi's bf16 planes.  x that is not
+ * that is not bf16, or D % 8 != 0, it includes the general form's sums over
+ * split columns, S * (M + 1) floats a token for at most 4194176 tokens (more run
+ * in chunks): on 256 CUs S <= 129 at few tokens, 5 at 16384, 3 at 32768 and 2
+ * from 65536 on; with less, the tokens run in chunks that fit, or in a slower
+ * form that needs only phi's bf16 planes.  x that is not
  * bf16, and x, phi, y or x_scaled that is not 16-byte aligned, run the general
  * form whatever phi is: ask with MHC_DTYPE_F32 then (less may be refused where
  * it does not hold phi's planes either).
